@@ -396,6 +396,18 @@ void launch_mmq_gguf_q4_k_q8k(void *tmp_fixup, const void *x, const void *y, voi
 void launch_mmq_gguf_q5_k_q8k(void *tmp_fixup, const void *x, const void *y, void *dst, int64_t ncols_x,
                               int64_t nrows_x, int64_t ncols_y, int64_t stride_row_x, int64_t stride_col_dst, int cc,
                               int nsm, int64_t smpbo, int warp_size, int type_dst, void *stream);
+/* launch_mmq_gguf_{q4_k,q6_k}_moe_glu: no counterpart in the reference, whose grouped route runs launch_mmq_gguf_<t>_moe
+ * for gate and for up and applies the GLU while it quantizes their outputs again.  Gate and up in one launch over the
+ * same expert-sorted activation tiles (either Q8_K layout): dst[m * stride_col_dst + n] = act(W_gate[e] . y_m) *
+ * (W_up[e] . y_m) for activation row m of expert e, in the activations' order (no ids_dst); activation as
+ * launch_mmq_quantize_glu_*.  For few rows per expert: returns 1, or 0 having launched nothing where the two launches
+ * are to be used (more than 32 rows an expert on average), or -1 with the error recorded. */
+int launch_mmq_gguf_q4_k_moe_glu(const void *x_gate, const void *x_up, const void *y, const int32_t *expert_bounds,
+                                 float *dst, int64_t ncols_x, int64_t nrows_x, int64_t ncols_dst, int64_t stride_row_x,
+                                 int64_t stride_col_dst, int64_t num_experts, int activation, void *stream);
+int launch_mmq_gguf_q6_k_moe_glu(const void *x_gate, const void *x_up, const void *y, const int32_t *expert_bounds,
+                                 float *dst, int64_t ncols_x, int64_t nrows_x, int64_t ncols_dst, int64_t stride_row_x,
+                                 int64_t stride_col_dst, int64_t num_experts, int activation, void *stream);
 /* launch_mmq_gguf_{q4_k,q5_k}_moe_q8k: no counterpart in the reference; launch_mmq_gguf_<t>_moe over `_q8k` tiles
  * (launch_mmq_quantize_q8k with the dispatch's row ids, or launch_mmq_quantize_glu_q8k_f32), the same results. */
 void launch_mmq_gguf_q4_k_moe_q8k(void *tmp_fixup, const void *x, const void *y, const int32_t *ids_dst,

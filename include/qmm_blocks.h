@@ -173,10 +173,11 @@ static inline int qmm_vec_dot_type(int t) { return qmm_block_size(t) == 32 ? QMM
 
 /* The decode / prefill boundary of QMatMul::forward, shared by the host layer and qmm_qmatmul_forward_noalloc: up to
  * this many activation rows take the decode launchers (fast_mmvq.rs TENSOR_CORE_MAX_ROWS = 16, re-derived for gfx950:
- * Q4_K, and Q6_K rows of at most 8192 values, stay on the decode launcher up to 32 rows, where its few-row MFMA
- * kernel still beats the prefill matmul), more the prefill matmul. */
+ * Q4_K and Q6_K stay on the decode launcher up to 32 rows, where its few-row MFMA kernel beats the prefill matmul:
+ * with their quantizers, at 24 rows, Q4_K 14336x4096 15.4 against 19.0 us, Q6_K 4096x14336 22.2 against 31.1), more the
+ * prefill matmul.  (Q6_K rows past 131072 values keep the prefill matmul, whose activations are the smaller.) */
 static inline int64_t qmm_max_decode_rows(int type, int64_t k) {
-  return type == QMM_TYPE_Q4K || (type == QMM_TYPE_Q6K && k <= 8192) ? 32 : 16;
+  return type == QMM_TYPE_Q4K || (type == QMM_TYPE_Q6K && k <= 131072) ? 32 : 16;
 }
 
 #endif

@@ -258,7 +258,7 @@ void fused_glu(const void *vx_gate, const void *vx_up, const void *vy, void *dst
   if (b == 0 || nrows_x == 0) return;
   hipStream_t s = (hipStream_t)stream;
   if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
-    if (b >= qmm_skinny_min_rows(T) &&
+    if (b >= qmm_skinny_min_rows(ncols_x) &&
         qmm_skinny_glu(T, out_type_of((const Out *)nullptr), vx_gate, vx_up, vy, dst, ncols_x, nrows_x, stride_col_y,
                        stride_col_dst, b, activation, s))
       return;
@@ -280,7 +280,7 @@ void fused_qkv(const void *vx_q, const void *vx_k, const void *vx_v, const void 
   if (b == 0 || nrows_q + nrows_k + nrows_v == 0) return;
   hipStream_t s = (hipStream_t)stream;
   if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
-    if (b >= qmm_skinny_min_rows(T)) {
+    if (b >= qmm_skinny_min_rows(ncols_x)) {
       const int ot = out_type_of((const Out *)nullptr);
       const void *w[3] = {vx_q, vx_k, vx_v};
       void *d[3] = {q_dst, k_dst, v_dst};

@@ -1325,7 +1325,7 @@ void mmq_moe_t(int type, void *tmp_fixup, const void *x, const void *y, const in
   const ActTile a = act_tile(y, ncols_dst, nsb);
   const dim3 grid((unsigned)((nrows_x + BN - 1) / BN), (unsigned)((ncols_max + BM - 1) / BM), (unsigned)num_experts);
   hipStream_t s = (hipStream_t)stream;
-  // a few rows per expert: the few-row kernel streams each expert's weights once, without 64-row tiles of padding
+  // a few rows per expert: the few-row kernel, which streams each expert's weights once
   const bool b32 = qmm_block_size(type) == 32;  // Q8_0, Q4_0, Q5_0: the Q8_0-layout kernel
   if (!b32 && F32D && qmm_skinny_moe(type, x, y, ids_dst, bounds, (float *)dst, ncols_x, nrows_x, w_row_bytes,
                                               ncols_dst, stride_col_dst, num_experts, s))
@@ -1433,6 +1433,9 @@ void mmq_moe_q8k(int type, void *tmp_fixup, const void *x, const void *y, const 
   hipStream_t s = (hipStream_t)stream;
   const uint8_t *w = (const uint8_t *)x;
   float *d = (float *)dst;
+  if (qmm_skinny_moe(type, x, y, ids_dst, bounds, d, ncols_x, nrows_x, w_row_bytes, ncols_dst, stride_col_dst,
+                     num_experts, s))
+    return;
   const bool small = (QMM_MOE_SMALL_AVG ? (ncols_dst + num_experts - 1) / num_experts : ncols_max) <= 32 ||
                      type == QMM_TYPE_Q5K;
   const int64_t ntiles = (nrows_x + BN - 1) / BN;
@@ -1451,6 +1454,27 @@ void mmq_moe_q8k(int type, void *tmp_fixup, const void *x, const void *y, const 
     kq_moe<wq4k, 2, true>(gridk, s, w, expert_bytes, nrows_x, w_row_bytes, a, bounds, ids_dst, nsb, splits, d,
                           stride_col_dst, part, ncols_dst);
   if (part) split_sum<out_f32>(part, splits, ncols_dst, nrows_x, d, stride_col_dst, ids_dst, s);
+}
+
+// launch_mmq_gguf_{q4_k,q6_k}_moe_glu
+int mmq_moe_glu(int type, const void *gate, const void *up, const void *y, const int32_t *bounds, float *dst,
+                int64_t ncols_x, int64_t nrows_x, int64_t ncols_dst, int64_t stride_row_x, int64_t stride_col_dst,
+                int64_t num_experts, int activation, void *stream, const char *who) {
+  if (!check_mmq(who, type, gate, ncols_x, nrows_x, stride_row_x) ||
+      !check_mmq(who, type, up, ncols_x, nrows_x, stride_row_x) || !check_act_bytes(who, ncols_x, ncols_dst))
+    return -1;
+  if (num_experts <= 0 || ncols_dst < 0 || stride_col_dst < nrows_x || num_experts > 65535 || activation < 0 ||
+      activation >= kGluActivations) {
+    qmm_set_error("%s: num_experts=%lld ncols_dst=%lld stride_col_dst=%lld activation=%d", who, (long long)num_experts,
+                  (long long)ncols_dst, (long long)stride_col_dst, activation);
+    return -1;
+  }
+  if (ncols_dst == 0) return 1;
+  return qmm_skinny_moe_glu(type, gate, up, y, bounds, dst, ncols_x, nrows_x,
+                            stride_row_x * (int64_t)qmm_type_size(type), ncols_dst, stride_col_dst, num_experts,
+                            activation, (hipStream_t)stream)
+             ? 1
+             : 0;
 }
 
 }  // namespace
@@ -1504,6 +1528,17 @@ QMM_DEFINE_MMQ_ENTRIES(q5_0, QMM_TYPE_Q5_0, true, _q8_0)
     mmq_moe_q8k(TYPE, tmp_fixup, x, y, ids_dst, expert_bounds, dst, ncols_x, nrows_x, ncols_dst, stride_row_x,     \
                 stride_col_dst, num_experts, ncols_max, nsm, stream, "mmq_" #t "_moe_q8k");                        \
   }
+#define QMM_DEFINE_MMQ_MOE_GLU(t, TYPE)                                                                            \
+  int launch_mmq_gguf_##t##_moe_glu(const void *x_gate, const void *x_up, const void *y, const int32_t *expert_bounds,  \
+                                    float *dst, int64_t ncols_x, int64_t nrows_x, int64_t ncols_dst,               \
+                                    int64_t stride_row_x, int64_t stride_col_dst, int64_t num_experts,             \
+                                    int activation, void *stream) {                                                \
+    return mmq_moe_glu(TYPE, x_gate, x_up, y, expert_bounds, dst, ncols_x, nrows_x, ncols_dst, stride_row_x,        \
+                       stride_col_dst, num_experts, activation, stream, "mmq_" #t "_moe_glu");                     \
+  }
+QMM_DEFINE_MMQ_MOE_GLU(q4_k, QMM_TYPE_Q4K)
+QMM_DEFINE_MMQ_MOE_GLU(q6_k, QMM_TYPE_Q6K)
+#undef QMM_DEFINE_MMQ_MOE_GLU
 QMM_DEFINE_MMQ_Q8K(q4_k, QMM_TYPE_Q4K)
 QMM_DEFINE_MMQ_Q8K(q5_k, QMM_TYPE_Q5K)
 #undef QMM_DEFINE_MMQ_Q8K

@@ -1044,7 +1044,7 @@ void plain_t(const void *vx, const void *vy, void *dst, int ncols_x, int nrows_x
   const uint8_t *x = (const uint8_t *)vx, *y = (const uint8_t *)vy;
   typename Out::T *d = (typename Out::T *)dst;
   if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
-    if (b >= qmm_skinny_min_rows(T) &&
+    if (b >= qmm_skinny_min_rows(ncols_x) &&
         qmm_skinny_decode(T, out_type_of((const Out *)nullptr), vx, vy, dst, ncols_x, nrows_x, stride_col_y,
                           stride_col_dst, b, s))
       return;
@@ -1222,7 +1222,7 @@ void tc_plain_t(const void *vx, const void *vy, void *dst, int ncols_x, int nrow
   if (!check_mmvq<T, kActSlots>(who, vx, ncols_x, nrows_x, ncols_x / 32, b)) return;
   if (b == 0) return;
   hipStream_t s = (hipStream_t)stream;
-  if (b >= qmm_skinny_min_rows(T) &&
+  if (b >= qmm_skinny_min_rows(ncols_x) &&
       qmm_skinny_tc(T, out_type_of((const Out *)nullptr), vx, vy, dst, ncols_x, nrows_x, stride_col_dst, b, s))
     return;
   typedef typename std::conditional<T == QMM_TYPE_Q4K, unit_q4k_tc, unit_q6k_tc>::type U;

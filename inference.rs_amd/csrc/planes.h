@@ -33,6 +33,16 @@ __device__ __forceinline__ void swap_lane_halves(uint32_t &lo, uint32_t &hi) {
 #endif
 }
 
+// v_permlane16_swap_b32 (gfx950): the odd rows of 16 lanes of a trade places with the even rows of b, so that a + b is
+// a plus the partner's a (lane ^ 16) in even rows, b plus the partner's b in odd rows
+__device__ __forceinline__ void swap_lane_rows(uint32_t &a, uint32_t &b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+#endif
+}
+
 // The two int8 planes of four weights w in [-4224, 4095]: lo and hi hold w + 128 of weights (0, 2) and (1, 3) in
 // their 16-bit lanes.  w + 128 = 256 wh + (wl + 128): wh is the high byte of the lane, wl its low byte less 128
 // (the low byte with its top bit flipped, as int8), so each plane is one byte permute.
@@ -417,9 +427,11 @@ __device__ __forceinline__ v4f mfma16_f16(v4h a, v4h b, v4f c) {
 
 // Q4_K: step t = 2p + h takes nibble h of bytes qs[64p + 16kg .. +16], i.e. values 128p + 64(kg/2) + 32h +
 // 16(kg%2) + (0..15) of sub-block 4p + 2(kg/2) + h.  Per lane per superblock: the 16-byte header and two 16-byte
-// chunks of nibbles.
+// chunks of nibbles.  The min term: lane group kg carries sub-blocks 4p + 2(kg/2) + {0, 1} with p = kg % 2, the ones
+// whose activation sums it can form from its own A fragments and its partner's (lane ^ 16).
 struct wq4k16 {
   static constexpr int kBytes = 144;
+  static constexpr int kPieces = 9;  // 16-byte pieces of a superblock (of its window) in LDS
   static constexpr int kShift = 3;
   static constexpr bool kMin = true;
   struct Raw {
@@ -428,44 +440,33 @@ struct wq4k16 {
   static __device__ __forceinline__ uint32_t act_offset(int t, int kg) {
     return 128 * (t >> 1) + 64 * (kg >> 1) + 32 * (t & 1) + 16 * (kg & 1);
   }
-  static __device__ __forceinline__ void load(rsrc_t rs, uint32_t row, uint32_t sb, int kg, Raw &r) {
-    const uint32_t o = row + sb * kBytes;
-    r.hdr = __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0);
-#pragma unroll
-    for (int p = 0; p < 2; p++) r.q[p] = __builtin_amdgcn_raw_buffer_load_b128(rs, o + 16 + 64 * p + 16 * kg, 0, 0);
+  // the superblock at p in LDS
+  static __device__ __forceinline__ void load_lds(const uint8_t *p, uint32_t, int kg, Raw &r) {
+    r.hdr = *(const u32x4 *)p;
+    r.q[0] = *(const u32x4 *)(p + 16 + 16 * kg);
+    r.q[1] = *(const u32x4 *)(p + 80 + 16 * kg);
   }
   struct Prep {
     uint32_t sh[4], sl[4];
     float d, dmin;
     v4h bmin;
   };
+  // get_scale_min_k4 (quantized/utils.rs:119-129) on the two sub-blocks of each half p that this lane group decodes:
+  // their scales' and mins' bytes come to the bottom of the header's three dwords with one shift each
   static __device__ __forceinline__ void prepare(const Raw &r, int kg, Prep &p) {
-    const uint32_t s[3] = {r.hdr.y, r.hdr.z, r.hdr.w};
-    auto byte = [&](int i) { return (s[i >> 2] >> (8 * (i & 3))) & 0xffu; };
-    uint32_t sc[8], m[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {  // get_scale_min_k4 (quantized/utils.rs:119-129)
-      sc[j] = j < 4 ? byte(j) & 63 : (byte(j + 4) & 0xf) | ((byte(j - 4) >> 6) << 4);
-      m[j] = j < 4 ? byte(j + 4) & 63 : (byte(j + 4) >> 4) | ((byte(j) >> 6) << 4);
-    }
-    const bool hi = kg >= 2;
+    const uint32_t sft = kg >= 2 ? 16 : 0;
+    const uint32_t q0 = r.hdr.y >> sft, q1 = r.hdr.z >> sft, q2 = r.hdr.w >> sft;
+    const uint32_t sc[2] = {q0 & 0x3f3fu, (q2 & 0x0f0fu) | ((q0 >> 2) & 0x3030u)};
+    const uint32_t m = (kg & 1) ? ((q2 >> 4) & 0x0f0fu) | ((q1 >> 2) & 0x3030u) : q1 & 0x3f3fu;
 #pragma unroll
     for (int t = 0; t < 4; t++) {
-      const int j = 4 * (t >> 1) + (t & 1);  // sub-block for kg < 2; kg >= 2 adds 2
-      const uint32_t v = hi ? sc[j + 2] : sc[j];
+      const uint32_t v = (t & 1) ? sc[t >> 1] >> 8 : sc[t >> 1] & 0xffu;
       p.sh[t] = v >> 3;
       p.sl[t] = v & 7;
     }
     p.d = f16_bits_to_f32(r.hdr.x & 0xffff);
     p.dmin = f16_bits_to_f32(r.hdr.x >> 16);
-    // min-term B of sub-blocks 2kg, 2kg + 1: (64 m0, 64 m1, m0, m1), min_frag's order
-    uint32_t m0 = m[0], m1 = m[1];
-#pragma unroll
-    for (int q = 1; q < 4; q++)
-      if (kg == q) {
-        m0 = m[2 * q];
-        m1 = m[2 * q + 1];
-      }
+    const uint32_t m0 = m & 0xffu, m1 = m >> 8;  // (64 m0, 64 m1, m0, m1), min_frag's order
     p.bmin = (v4h){(_Float16)(float)(64 * m0), (_Float16)(float)(64 * m1), (_Float16)(float)m0, (_Float16)(float)m1};
   }
   static __device__ __forceinline__ void planes(const Raw &r, const Prep &p, int t, v4i &b1, v4i &b2, int) {
@@ -484,32 +485,39 @@ struct wq4k16 {
 // the 2-bit fields 2q, q = 2(t%2) + kg/2, of qh[32(t/2) + 16(kg%2) ..], scale sc[4t + kg].
 struct wq6k16 {
   static constexpr int kBytes = 210;
+  static constexpr int kPieces = 14;
   static constexpr int kShift = 8;  // split256
   static constexpr bool kMin = false;
   // chunks kept unaligned until prepare(), as in wq6k
   typedef wq6k::Chunk Chunk;
   struct Raw {
     Chunk ql[2], qh[2], sc;
-    uint32_t off;
-    uint32_t d;
+    uint32_t off, d;
   };
   static __device__ __forceinline__ uint32_t act_offset(int t, int kg) { return 64 * t + 16 * kg; }
-  static __device__ __forceinline__ void load(rsrc_t rs, uint32_t row, uint32_t sb, int kg, Raw &r) {
-    const uint32_t o = row + sb * kBytes, off = o & 3, a4 = o - off;
+  // the superblock whose window (224 bytes from the dword holding its first byte) is at p in LDS, off = its start (0 or
+  // 2).  (Read where it lies, 2-byte aligned, instead: LDS reads of 16 bytes off their alignment measured slower, the
+  // 4096x14336 matvec at 4 rows 13.7 -> 14.5 us.)
+  static __device__ __forceinline__ void load_lds(const uint8_t *p, uint32_t off, int kg, Raw &r) {
+    auto ld = [&](int o, Chunk &c) {
+      c.v = *(const u32x4 *)(p + o);
+      c.e = *(const uint32_t *)(p + o + 16);
+    };
 #pragma unroll
     for (int x = 0; x < 2; x++) {
-      wq6k::ld16(rs, a4, 64 * x + 16 * kg, r.ql[x]);
-      wq6k::ld16(rs, a4, 128 + 32 * x + 16 * (kg & 1), r.qh[x]);
+      ld(64 * x + 16 * kg, r.ql[x]);
+      ld(128 + 32 * x + 16 * (kg & 1), r.qh[x]);
     }
-    wq6k::ld16(rs, a4, 192, r.sc);  // the fifth dword may end past the last row: it then reads as 0, unused
+    ld(192, r.sc);
     r.off = off;
-    r.d = __builtin_amdgcn_raw_buffer_load_b16(rs, o + 208, 0, 0);
+    r.d = *(const uint16_t *)(p + 208 + off);
   }
   struct Prep {
     int sc[4];
     float d, dmin;
     v4h bmin;
-    uint32_t ql[2][4], qh[2][4];  // realigned
+    uint32_t ql[2][4];
+    uint32_t qh[2][4];  // this lane group's fields: bits 0..1 of every byte for even t, bits 4..5 for odd t
   };
   static __device__ __forceinline__ void prepare(const Raw &r, int kg, Prep &p) {
     uint32_t sc[4];
@@ -517,25 +525,28 @@ struct wq6k16 {
 #pragma unroll
     for (int t = 0; t < 4; t++)  // byte 4t + kg of the 16 scales = byte kg of dword t
       p.sc[t] = (int)(int8_t)((sc[t] >> (8 * kg)) & 0xff);
+    const uint32_t sft = 2 * (kg >> 1);
 #pragma unroll
     for (int x = 0; x < 2; x++) {
       wq6k::words(r.ql[x], r.off, p.ql[x]);
       wq6k::words(r.qh[x], r.off, p.qh[x]);
+#pragma unroll
+      for (int i = 0; i < 4; i++) p.qh[x][i] >>= sft;
     }
     p.d = f16_bits_to_f32(r.d);
     p.dmin = 0.0f;
     p.bmin = (v4h){};
   }
-  static __device__ __forceinline__ void planes(const Raw &r, const Prep &p, int t, v4i &b1, v4i &b2, int kg) {
-    (void)r;
-    const uint32_t *ql = p.ql[t >> 1], *qh = p.qh[t >> 1];
-    const int nsh = 4 * (t & 1), hsh = 4 * (t & 1) + 2 * (kg >> 1);
+  static __device__ __forceinline__ void planes(const Raw &, const Prep &p, int t, v4i &b1, v4i &b2, int) {
     const s2 sc2 = {(short)p.sc[t], (short)p.sc[t]};
     const s2 c2 = (s2){128, 128} - (s2){32, 32} * sc2;  // (q6 - 32) sc + 128 = q6 sc + c2
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      s2 lo, hi;
-      q6_lanes(ql[i] >> nsh, qh[i], hsh, lo, hi);
+      const uint32_t l = (t & 1) ? p.ql[t >> 1][i] >> 4 : p.ql[t >> 1][i];
+      const uint32_t h = (t & 1) ? p.qh[t >> 1][i] : p.qh[t >> 1][i] << 4;
+      const uint32_t v6 = (l & 0x0f0f0f0fu) | (h & 0x30303030u);
+      const s2 lo = __builtin_bit_cast(s2, v6 & 0x00ff00ffu);
+      const s2 hi = __builtin_bit_cast(s2, (v6 >> 8) & 0x00ff00ffu);
       split256(lo * sc2 + c2, hi * sc2 + c2, b1, b2, i);  // w + 128
     }
   }

@@ -492,7 +492,8 @@ void fused_ffn(const QMatMul &gate, const QMatMul &up, const QMatMul &down, cons
   const GgmlDType t = g.dtype();
   const int ordinal = g.device().ordinal;
   hip_check(hipSetDevice(ordinal), "hipSetDevice");
-  if (rows <= QMatMul::kMaxDecodeRows) {
+  // (17 to 32 rows, 2 x Q4_K 14336x4096 at 24: the fused-GLU matvec 21.0 us, the two prefill matmuls 2 x 14)
+  if (rows <= (t == GgmlDType::Q8_0 ? QMatMul::kMaxDecodeRows : QMatMul::kMaxFewRows)) {
     // decode: one activation quantization, the fused-GLU matvec, then down on act(gate) * up
     const int64_t kp = pad_to(hidden, act_block(t));
     Carver c;
@@ -571,7 +572,8 @@ void MoeExperts::forward(const float *xs, int64_t tokens, const int32_t *ids, co
   const int ordinal = gate_->device().ordinal;
   hip_check(hipSetDevice(ordinal), "hipSetDevice");
   const GgmlDType tg = gate_->dtype(), td = down_->dtype();
-  const bool grouped = force_grouped || tokens > kIndexedMaxTokens;
+  const bool few_row = tg != GgmlDType::Q8_0 && td != GgmlDType::Q8_0;  // (the others are Q4_K and Q6_K)
+  const bool grouped = force_grouped || tokens > (few_row ? kIndexedMaxTokensFewRow : kIndexedMaxTokens);
   if (!grouped) {
     // decode: fused gate/up matvec per routed pair, then down with the weighted sum over slots folded in
     const int64_t kp1 = pad_to(hidden, act_block(tg)), kp2 = pad_to(inter, act_block(td));
@@ -619,17 +621,29 @@ void MoeExperts::forward(const float *xs, int64_t tokens, const int32_t *ids, co
   prefill_quantizer(tg)(xs, src, ws + o_x, 0, hidden, hidden, hidden * tokens, hidden * tokens, kp1, pairs, 1, 1,
                         stream);
   abi_check("MoE grouped (quantize x)");
-  for (int which = 0; which < 2; which++) {
+  // few rows per expert: gate and up in one launch, act(gate) * up in the experts' row order
+  const int fused =
+      tg == GgmlDType::Q8_0
+          ? 0
+          : (tg == GgmlDType::Q4K ? launch_mmq_gguf_q4_k_moe_glu : launch_mmq_gguf_q6_k_moe_glu)(
+                gate_->device_ptr(), up_->device_ptr(), ws + o_x, bounds, (float *)(ws + o_g), hidden, inter, pairs,
+                hidden / (int64_t)block_size(tg), inter, E, activation_, stream);
+  abi_check("MoE grouped (gate/up GLU)");
+  for (int which = 0; which < 2 && !fused; which++) {
     const QTensor &w = which == 0 ? *gate_ : *up_;
     prefill_matmul_moe(tg)(ws + o_fix, w.device_ptr(), ws + o_x, tok, bounds, ws + (which == 0 ? o_g : o_u), hidden,
                            inter, pairs, hidden / (int64_t)block_size(tg), inter, E, pairs, 0, nsm, 160 * 1024, 64,
                            stream);
     abi_check("MoE grouped (gate/up)");
   }
-  (act_q8_0(td)      ? launch_mmq_quantize_glu_q8_0_f32
-   : prefill_q8k(td) ? launch_mmq_quantize_glu_q8k_f32
-                     : launch_mmq_quantize_glu_q8_1_DS4_f32)((const float *)(ws + o_g), (const float *)(ws + o_u), tok,
-                                                             ws + o_mq, inter, inter, kp2, pairs, activation_, stream);
+  if (fused)
+    prefill_quantizer(td)(ws + o_g, nullptr, ws + o_mq, 0, inter, inter, inter * pairs, inter * pairs, kp2, pairs, 1, 1,
+                          stream);
+  else
+    (act_q8_0(td)      ? launch_mmq_quantize_glu_q8_0_f32
+     : prefill_q8k(td) ? launch_mmq_quantize_glu_q8k_f32
+                       : launch_mmq_quantize_glu_q8_1_DS4_f32)((const float *)(ws + o_g), (const float *)(ws + o_u), tok,
+                                                               ws + o_mq, inter, inter, kp2, pairs, activation_, stream);
   abi_check("MoE grouped (GLU + quantize)");
   // down, then the weighted sum over each token's routes as its own launch: folded into the down projection (a
   // counter per token and column tile, the workgroup completing it summing the routes) it measured 381 us against

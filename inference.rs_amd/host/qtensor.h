@@ -116,12 +116,9 @@ class QTensor {
 class QMatMul {
  public:
   static constexpr int64_t kMaxDecodeRows = 16;  // fast_mmvq.rs TENSOR_CORE_MAX_ROWS, re-derived for gfx950
-  // Q4_K, and Q6_K with rows of at most kMaxFewRowK values, stay on the decode launcher up to 32 rows: its few-row
-  // MFMA kernel streams the weight once for all of them and measured faster than the prefill tile there on MI355X
-  // (Q4_K 4096x4096 at 32 rows 10.4 against 13.2 us; Q6_K 4096x14336 is the exception, 34.6 against 31.7 us, as
-  // the reference keeps Q6_K's widest rows on MMQ, fast_mmvq.rs:1838-1881)
+  // Q4_K and Q6_K stay on the decode launcher up to 32 rows (qmm_max_decode_rows): its few-row MFMA kernel streams the
+  // weight once for all of them
   static constexpr int64_t kMaxFewRows = 32;
-  static constexpr int64_t kMaxFewRowK = 8192;
 
   explicit QMatMul(std::shared_ptr<QTensor> w);
   const QTensor &weight() const { return *w_; }
@@ -152,7 +149,7 @@ class QMatMul {
 
 // fast_mmq::fused_ffn (gguf/fast_mmq.rs:883-899): ys[rows, hidden] = down(act(gate(xs)) * up(xs)) for f32 xs
 // [rows, hidden], gate and up [inter, hidden] of one type, down [hidden, inter].  Gate and up read one activation
-// quantization (shared_lhs, fast_mmq.rs:537-602).  Up to QMatMul::kMaxDecodeRows rows they run as the fused-GLU
+// quantization (shared_lhs, fast_mmq.rs:537-602).  Up to 16 rows (Q4_K and Q6_K gate / up: 32) they run as the fused-GLU
 // matvec (launch_mmvq_gguf_<t>_f32_fused_glu, which stores act(gate) * up) and down as QMatMul::forward; above, as
 // two prefill matmuls whose f32 outputs go through down.down_from_glu.
 void fused_ffn(const QMatMul &gate, const QMatMul &up, const QMatMul &down, const float *xs, int64_t rows,
@@ -164,6 +161,11 @@ void fused_ffn(const QMatMul &gate, const QMatMul &up, const QMatMul &down, cons
 class MoeExperts {
  public:
   static constexpr int64_t kIndexedMaxTokens = 8;      // backends.rs:25 INDEXED_MMVQ_MAX_TOKENS
+  // Experts of Q4_K / Q6_K, whose grouped route has the few-row kernel, take it from 5 tokens on: an expert's weights are
+  // then read once for all of its rows.  Indexed / grouped on MI355X, 8 x Q4_K of 14336, top-2, at 1 / 2 / 4 / 8 tokens:
+  // 39 / 80 / 136 / 239 and 64 / 107 / 121 / 151 us (4 tokens routed to more experts: 130 and 136); 16 Q4_K / Q6_K of
+  // 4096, top-4: 33 / 52 / 113 / 204 and 50 / 63 / 92 / 118 us.
+  static constexpr int64_t kIndexedMaxTokensFewRow = 4;
   static constexpr int64_t kGroupedMinTokens = 32;     // backends.rs:22 GROUPED_PREFILL_MIN_TOKENS
 
   MoeExperts(std::shared_ptr<QTensor> gate, std::shared_ptr<QTensor> up, std::shared_ptr<QTensor> down,
