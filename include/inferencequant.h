@@ -532,7 +532,7 @@ void moe_router_topk_f16(const void *logits, float *weights, uint32_t *ids, cons
  * QMatMul::forward (qmm_qmatmul_forward in qmm_host.h, whose per-thread workspace grows with hipMalloc) with the same
  * routes and kernels: ys[rows, n] = xs[rows, k] . W^T, W = n rows of GGUF blocks of type wtype (8 q8_0, 12 q4_k,
  * 14 q6_k, 2 q4_0, 6 q5_0, 13 q5_k, 23 iq4_xs) padded as QTensor pads them; xs and ys device pointers of in_dtype
- * (0 f32, 1 f16, 30 bf16).  Quantized activations and split-K planes live in one 32 MiB device array of the library,
+ * (0 f32, 1 f16, 30 bf16).  Quantized activations and split-K planes live in one 80 MiB device array of the library,
  * held by each device it runs on until the process ends; the quantized activations must fit in its 16 MiB
  * activation part (rows * ceil(k / 256) * 292 bytes, 272 for the 32-value block types, above 16 rows; rows * k / 256 *
  * 292 or rows * k / 32 * 34 bytes at 16 rows or fewer), else nothing is launched and the call returns -1 with

@@ -180,4 +180,18 @@ static inline int64_t qmm_max_decode_rows(int type, int64_t k) {
   return type == QMM_TYPE_Q4K || (type == QMM_TYPE_Q6K && k <= 131072) ? 32 : 16;
 }
 
+/* The `nsm` (fixup buffer size / 65536 bytes) that QMatMul::forward and qmm_qmatmul_forward_noalloc give a prefill
+ * launch: a K-quant prefill may split K until its 128-row tiles of 256 weight rows fill the compute units, in up to 64 MiB
+ * of f32 planes.  (At 512 rows Q6_K 4096x14336 takes four planes of 8 MiB; the reference's buffer, 16 MiB, holds two, and
+ * half the compute units would have no tile.) */
+#define QMM_MAX_FIXUP_BYTES ((int64_t)64 << 20)
+static inline int qmm_fixup_nsm(int nsm, int type, int64_t n, int64_t k, int64_t rows) {
+  if (qmm_block_size(type) != 256 || rows <= 32) return nsm;
+  const int64_t tiles = (rows + 127) / 128 * ((n + 255) / 256), nsb = k / 256;
+  int64_t s = 1;
+  while (tiles * s < nsm && nsb / (s * 2) >= 4 && 2 * s * rows * n * 4 <= QMM_MAX_FIXUP_BYTES) s *= 2;
+  const int64_t want = s > 1 ? (s * rows * n * 4 + 65535) / 65536 : 0;
+  return want > nsm ? (int)want : nsm;
+}
+
 #endif

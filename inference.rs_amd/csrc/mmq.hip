@@ -974,6 +974,203 @@ __device__ __forceinline__ void tile_of(int64_t mtiles, int64_t ntiles, int64_t 
   nt = tile / mtiles;
 }
 
+// ------------------------------------------------------------------------------------------ K-quant, wide tiles
+
+template <class WT>
+struct Wide {  // the weight policy of the wide kernel (two planes)
+  typedef WT T;
+};
+template <>
+struct Wide<wq5k> {
+  typedef wq5k2 T;
+};
+
+// The K-quant prefill from 65 activation rows on: a workgroup of 8 waves x 32 weight rows (256) against 32 TM = 128 (or
+// 64) activation rows, one workgroup per CU, two waves per SIMD.  The same exact integer arithmetic as mmq_kq_tile.
+//
+// What bounds it: power.  At M = 512, 14336x4096, the kernel runs at 1.8 to 2.0 GHz (2.35 at one wave per SIMD), and
+// variants that took fewer cycles ran at a lower clock in the same time; the matrix core is busy 60% of the cycles.  So the
+// aim is fewer operations per output: a wave builds a superblock's planes once for all 128 rows (the 64-row kernel: for
+// 64) and keeps them in registers, then takes the activation tiles one after another, so only one tile's integer sums
+// are live (the order that kept every tile's sums live had no registers for 128 rows at two waves per SIMD).
+// Both waves of a SIMD would build planes at the same time after each barrier and multiply at the same time after that;
+// the second half of the workgroup (waves w and w + 4 share a SIMD) builds the next superblock's planes after its tiles
+// instead, so one wave's vector work falls into the other's MFMAs.  The next superblock's DMA loads are issued in thirds
+// after the first three tiles' MFMAs: issued together at the step's start, 88 of them per CU at 16 addresser cycles each,
+// every wave stalled on its own.  Activations: two LDS stages shared by the waves.  Weights: each wave's 32 rows in a
+// stage of its own, which it reloads once the superblock is in its registers.
+// MI355X, M = 512: Q4_K 14336x4096 90 -> 70 us, Q6_K 4096x14336 113 -> 79 us (without the staggered halves 71 and 81;
+// MFMA operands read into registers of their own a tile ahead, 76 and 83: the wider code ran at a higher clock in more
+// cycles; one wave per SIMD 90 and 100).
+template <class WT, class Out, int TM, bool S16>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mmq_wide(
+    const uint8_t *__restrict__ W, int64_t nrows_w, int64_t w_row_bytes, ActTile a, int64_t mrows, int64_t nsb,
+    int64_t splits, typename Out::T *__restrict__ dst, int64_t ldd, float *__restrict__ part) {
+  constexpr int NW = 8, BMt = 32 * TM, BNt = 32 * NW;
+  constexpr bool kWhole = WT::kBytes % 16 == 0;                              // superblocks of whole 16-byte pieces
+  constexpr int P = kWhole ? WT::kBytes / 16 : (WT::kBytes + 3 + 15) / 16;   // pieces of a superblock (of its window)
+  constexpr int SB = S16 ? 32 : 16;                                          // bytes of sums per row and superblock
+  constexpr int QS = BMt * 256, SBB = WT::kMin ? BMt * 32 : 0, AST = QS + SBB + BMt * 4;  // stage: rows, sums, scales
+  constexpr int WB = 32 * P * 16, LW = (32 * P + 63) / 64;                   // a wave's weights and their loads
+  constexpr int LQ = BMt * 16 / (64 * NW);                                   // a wave's loads of rows
+  static_assert(SB * BMt / 16 <= 64 * NW && BMt / 4 <= 64, "one load of sums per wave, one of scales");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * AST + NW * WB];
+
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5,
+            li = lane & 31;
+  int64_t mt, nt, split;
+  tile_of((mrows + BMt - 1) / BMt, (nrows_w + BNt - 1) / BNt, splits, mt, nt, split);
+  const int64_t m0 = mt * BMt, n0 = nt * BNt + 32 * wave, per = (nsb + splits - 1) / splits, rows = a.rows;
+  const int sb0 = (int)(split * per), sb1 = (int)(sb0 + per < nsb ? sb0 + per : nsb);
+  if (sb0 >= sb1) return;
+
+  const rsrc_t ra = make_rsrc(a.qs, nsb * rows * (260 + SB));
+  // this wave's weight rows, from the dword that holds the first byte to the end of the dword that holds the last
+  const int64_t rh = nrows_w - n0 < 32 ? nrows_w - n0 : 32;  // (none: an empty resource, zeros)
+  const uintptr_t wt = (uintptr_t)(W + (rh > 0 ? n0 : 0) * w_row_bytes);
+  const uint32_t dl = (uint32_t)(wt & 3);
+  const rsrc_t rw = make_rsrc((const uint8_t *)(wt - dl), rh > 0 ? (rh * w_row_bytes + dl + 3) & ~(int64_t)3 : 0);
+  uint8_t *const wl = lds + 2 * AST + wave * WB;
+  uint32_t wpc[LW], aq[LQ];
+#pragma unroll
+  for (int i = 0; i < LW; i++) {  // piece 64 i + lane: row C / P, 16-byte piece C % P
+    const int C = 64 * i + lane, row = C / P;
+    wpc[i] = (uint32_t)(row * w_row_bytes) + 16 * (uint32_t)(C - row * P) + dl;
+  }
+#pragma unroll
+  for (int i = 0; i < LQ; i++) {  // row r's chunk c at chunk slot c ^ (r % 16)
+    const int L = 64 * (NW * i + wave) + lane, r = L >> 4, c = (L & 15) ^ (r & 15);
+    aq[i] = (uint32_t)((m0 + r) * 256 + 16 * c);
+  }
+  auto dma = [&](rsrc_t r, uint8_t *p, uint32_t off, uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)p, 16, off, soff, 0, 0);
+#endif
+  };
+  // load k of superblock sb: the weights' LW (whole superblocks: the superblock's offset is uniform and a row past the end
+  // fails the range check by its own offset; else the window's dword, checked whole), then the activations' LQ of rows,
+  // the sums, the scales (rows past the channel read as zeros or the next section, and are not stored)
+  auto issue = [&](int sb, int u, int k) {
+    uint8_t *const st = lds + u * AST;
+    const uint32_t sr = (uint32_t)(sb * rows), os = (uint32_t)sb * WT::kBytes;
+    if (k < LW) {
+      if (64 * k + 64 <= 32 * P || lane < 32 * P - 64 * k)
+        dma(rw, wl + 1024 * k, kWhole ? wpc[k] : (wpc[k] + os) & ~3u, kWhole ? os : 0u);
+    } else if (k < LW + LQ) {
+      dma(ra, st + 1024 * (NW * (k - LW) + wave), aq[k - LW] + 256 * sr, 0);
+    } else if (k == LW + LQ) {
+      if (WT::kMin && 64 * wave < SB * BMt / 16)
+        dma(ra, st + QS + 1024 * wave, (uint32_t)(nsb * rows * 260 + m0 * SB + 16 * (64 * wave + lane)) + SB * sr, 0);
+    } else if (wave == NW - 1 && lane < BMt / 4) {
+      dma(ra, st + QS + SBB, (uint32_t)(nsb * rows * 256 + m0 * 4 + 16 * lane) + 4 * sr, 0);
+    }
+  };
+  constexpr int kIssues = LW + LQ + 2;
+
+  uint32_t qoff[8];  // this lane's A fragments: row 32t + li, chunk WT::chunk(j, g)
+#pragma unroll
+  for (int j = 0; j < 8; j++) qoff[j] = 256 * li + 16 * (WT::chunk(j, g) ^ (li & 15));
+  const uint32_t wo = (uint32_t)((li < rh ? li : 0) * w_row_bytes) + dl;
+  v16f fa[TM];
+#pragma unroll
+  for (int t = 0; t < TM; t++) fa[t] = (v16f){};
+  v4i b1[8], b2[8];
+  typename WT::Prep p;
+  auto decode = [&](int sb) {
+    typename WT::Raw raw;
+    WT::template load_lds<16>(wl + 16 * P * li, kWhole ? 0u : (wo + (uint32_t)sb * WT::kBytes) & 3u, g, raw);
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage is reloaded from here on
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (WT::kMin)
+      WT::template prepare<S16>(raw, g, p);
+    else
+      WT::prepare(raw, g, p);
+#pragma unroll
+    for (int j = 0; j < 8; j++) WT::planes(raw, p, j, b1[j], b2[j]);
+#pragma unroll
+    for (int j = 0; j < 8; j++) __asm__ volatile("" : "+v"(b1[j]), "+v"(b2[j]));
+  };
+
+#pragma unroll
+  for (int k = 0; k < kIssues; k++) issue(sb0, 0, k);
+  const bool late = wave >= NW / 2;
+  if (late) {
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    decode(sb0);
+  }
+  for (int sb = sb0; sb < sb1; sb++) {
+    const int u = (sb - sb0) & 1;
+    dma_barrier<0>();  // the stage of sb has landed, every wave is done with the other
+    if (!late) decode(sb);
+    const uint8_t *slot = lds + u * AST;
+#pragma unroll
+    for (int t = 0; t < TM; t++) {
+      v16i acc1 = (v16i){}, acc2 = (v16i){};
+      v4i av[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) av[j] = *(const v4i *)(slot + 8192 * t + qoff[j]);
+      // (a wave in its MFMAs gets the issue slots first)
+      __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        acc1 = mfma_i8(av[j], b1[j], acc1);
+        acc2 = mfma_i8(av[j], b2[j], acc2);
+      }
+      v16f fmin = (v16f){};
+      if (WT::kMin && S16) {
+        fmin = mfma_f16(*(const v8h *)(slot + QS + (32 * t + li) * 32 + 16 * g), p.bmin, fmin);
+      } else if (WT::kMin) {
+        const u32x2 sm = *(const u32x2 *)(slot + QS + (32 * t + li) * 16 + 8 * g);
+        fmin = mfma_f16(min_frag(sm.x, sm.y), p.bmin, fmin);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      constexpr int kParts = TM < 3 ? TM : 3;
+      if (t < kParts && sb + 1 < sb1) {
+#pragma unroll
+        for (int k = 0; k < kIssues; k++)
+          if (k * kParts / kIssues == t) issue(sb + 1, u ^ 1, k);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const v4f dy4 = *(const v4f *)(slot + QS + SBB + 4 * (32 * t + 8 * q + 4 * g));  // rows 8q + 4g + i
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int r = 4 * q + i;
+          float v = p.d * (float)((acc1[r] << WT::kShift) + acc2[r]);
+          if (WT::kMin) v = __builtin_fmaf(-p.dmin, fmin[r], v);
+          fa[t][r] = __builtin_fmaf(dy4[i], v, fa[t][r]);
+        }
+      }
+      // (formed here: left alone, the compiler moves the scaling on and keeps the integer sums in registers)
+      __asm__ volatile("" : "+v"(fa[t]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (late && sb + 1 < sb1) {
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      decode(sb + 1);
+    }
+  }
+
+  const int64_t n = n0 + li;
+  if (n >= nrows_w) return;
+  const int64_t ld = part ? nrows_w : ldd;
+  const int mleft = (int)(mrows - m0 < BMt ? mrows - m0 : BMt) - 4 * g;  // rows left from this lane's first
+  auto put = [&](auto *base, auto st) {
+    auto *q = base + (m0 + 4 * g) * ld + n;
+#pragma unroll
+    for (int t = 0; t < TM; t++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {  // row 32t + 8 (r / 4) + 4g + r % 4
+        if (32 * t + 8 * (r >> 2) + (r & 3) < mleft) st(q, fa[t][r]);
+        q += (r & 3) == 3 ? 5 * ld : ld;
+      }
+  };
+  if (part)  // split K: this split's partial sums (summed by k_split_sum)
+    put(part + split * mrows * nrows_w, [](float *q, float v) { *q = v; });
+  else
+    put(dst, [](typename Out::T *q, float v) { Out::store(q, 0, v); });
+}
+
 ActTile act_tile(const void *y, int64_t rows, int64_t nsb) {
   ActTile a;
   a.qs = (const uint8_t *)y;
@@ -1122,36 +1319,79 @@ int64_t k_splits(int64_t tiles, int64_t nsb, int64_t rows, int64_t cols, const v
   return s;
 }
 
-// Waves (weight rows / 32) per workgroup of the plain K-quant prefill from 64 activation rows per wave on (32-row
-// tiles keep 4: their per-wave DMA share would not be uniform over 8).  Measured on MI355X for Q4_K at M = 512 with
-// the weights staged in LDS: 8 waves 95.6 us, 4 waves 90.9 us -- a workgroup's waves run in lockstep between its
-// barriers, and two 4-wave workgroups per CU let one's VALU epilogue overlap the other's MFMAs.
-#ifndef QMM_KQ_WAVES
-#define QMM_KQ_WAVES 4
-#endif
+// The plain K-quant prefill's choice between its kernels, by the time a simple model gives each: a launch of `tiles`
+// output tiles over `splits` of K runs in rounds of the workgroups the chip holds, each round taking `us` per superblock
+// of K (a last round that leaves CUs idle or half idle less), after about 5 us of start and end; a split K adds its
+// planes' traffic and the summing launch.
+struct KqForm {
+  int tm, cols, per_cu;  // activation rows / 32 and weight rows of a tile, workgroups per CU
+  bool wide;
+  double us;
+};
+// us per round and superblock on MI355X.  Measured against it, us, 14336x4096 at 256 / 333 / 512 / 1024 rows: Q4_K 64-row
+// tiles 41 / 68 / 78 / 153, wide 54 / 56 / 65 / 127; Q6_K 128-row tiles 60 / 111 / 113 / 222, wide 72 / 74 / 78 / 156; Q5_K
+// 32-row tiles 71 / 94 / 128 / 261, wide 69 / 72 / 76 / 153; 4096x14336 at 512 rows: Q4_K 85 and 75, Q6_K 114 and 91, Q5_K
+// 133 and 86 (four planes).
+template <class WT>
+constexpr KqForm kq_form(int i) {
+  constexpr bool q4 = WT::kMin && WT::kPlanes == 2, q5 = WT::kPlanes == 3, q6 = WT::kBytes == 210;
+  return i == 0   ? KqForm{1, 128, 2, false, 2.2}  // up to 32 rows; Q5_K at any
+         : i == 1 ? KqForm{2, 128, q4 ? 2 : 1, false, q4 ? 2.4 : q6 ? 3.9 : 1.7}
+         : i == 2 ? KqForm{4, 128, 1, false, q6 ? 3.5 : 3.15}
+         : i == 3 ? KqForm{2, 256, 1, true, q4 ? 2.6 : q6 ? 3.9 : 3.4}
+                  : KqForm{4, 256, 1, true, q4 ? 3.75 : q6 ? 4.7 : 4.6};
+}
+inline double kq_us(const KqForm &f, int64_t tiles, int64_t splits, int64_t nsb, int64_t rows, int64_t cols) {
+  const int64_t cus = qmm_device_cus(), slots = f.per_cu * cus, full = tiles * splits / slots, rest = tiles * splits % slots;
+  const double last = rest == 0 ? 0 : f.per_cu == 2 ? (rest <= cus ? 0.6 : 1) : 0.8 + 0.2 * (double)rest / (double)cus;
+  return 5 + ((double)full + last) * (double)qmm_ceil_div(nsb, splits) * f.us +
+         (splits > 1 ? 3 + 1.5e-6 * (double)(splits * rows * cols) : 0);
+}
 
 template <class WT, class Out, bool S16 = false>
 void launch_kq(const uint8_t *w, int64_t nrows_x, int64_t w_row_bytes, const ActTile &a, int64_t ncols_y, int64_t nsb,
                typename Out::T *d, int64_t ldd, void *fixup, int nsm, hipStream_t s) {
-  // activation rows per wave: the smallest of 32, 64, 128 that covers the batch
-  const int tm = ncols_y <= 32 || kq_tm_max<WT>() < 2 ? 1 : ncols_y <= 64 || kq_tm_max<WT>() < 4 ? 2 : 4;
-  // (8 waves per workgroup fit where one wave needs at most 256 registers: Q4_K at 64 rows; Q6_K / IQ4_XS take 128
-  // rows at one wave per SIMD and keep 4)
-  constexpr int NW = WT::kMin && kq_tm_max<WT>() == 2 ? QMM_KQ_WAVES : 4;
-  const int nw = tm == 1 ? 4 : NW;
-  const int64_t ntiles = (nrows_x + 32 * nw - 1) / (32 * nw);
-  const int64_t tiles = ((ncols_y + 32 * tm - 1) / (32 * tm)) * ntiles;
-  const int64_t splits = k_splits(tiles, nsb, ncols_y, nrows_x, fixup, nsm);
+  // without the wide kernel, the smallest of 32, 64, 128 activation rows that covers the batch, split over as many planes
+  // as the reference's fixup buffer holds
+  KqForm f = kq_form<WT>(ncols_y <= 32 || kq_tm_max<WT>() < 2 ? 0 : ncols_y <= 64 || kq_tm_max<WT>() < 4 ? 1 : 2);
+  int64_t tiles = qmm_ceil_div(ncols_y, 32 * f.tm) * qmm_ceil_div(nrows_x, f.cols);
+  int64_t splits = k_splits(tiles, nsb, ncols_y, nrows_x, fixup, nsm < qmm_device_cus() ? nsm : qmm_device_cus());
+  if (ncols_y > 32) {
+    double best = kq_us(f, tiles, splits, nsb, ncols_y, nrows_x);
+    const int64_t planes = fixup && (uintptr_t)fixup % 16 == 0
+                               ? (int64_t)(nsm > 0 ? nsm : qmm_device_cus()) * 65536 / (4 * ncols_y * nrows_x)
+                               : 1;
+    // (a split wide form only where the model is clear: its planes' cost is the less certain part)
+    const double one = 0.97 * best, more = 0.9 * best;
+    for (int i = 3; i <= 4; i++) {
+      const KqForm c = kq_form<WT>(i);
+      const int64_t t = qmm_ceil_div(ncols_y, 32 * c.tm) * qmm_ceil_div(nrows_x, c.cols);
+      for (int64_t sp = 1; sp == 1 || (sp <= planes && nsb / sp >= 4); sp *= 2) {
+        const double us = kq_us(c, t, sp, nsb, ncols_y, nrows_x);
+        if (us < best && us < (sp == 1 ? one : more) && (sp - 1) * qmm_ceil_div(nsb, sp) < nsb) {
+          f = c;
+          tiles = t;
+          splits = sp;
+          best = us;
+        }
+      }
+    }
+  }
   float *part = splits > 1 ? (float *)fixup : nullptr;
   const dim3 grid((unsigned)(tiles * splits));
-  if (tm == 1) {
+  typedef typename Wide<WT>::T WW;
+  if (f.wide && f.tm == 2) {
+    k_mmq_wide<WW, Out, 2, S16><<<grid, 512, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
+  } else if (f.wide) {
+    k_mmq_wide<WW, Out, 4, S16><<<grid, 512, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
+  } else if (f.tm == 1) {
     k_mmq_kq<WT, Out, 1, 4, S16><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
-  } else if (tm == 2) {
-    k_mmq_kq<WT, Out, 2, NW, S16><<<grid, 64 * NW, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd,
-                                                          part);
-  } else if constexpr (kq_tm_max<WT>() >= 4) {  // (not instantiated where it cannot be chosen)
-    k_mmq_kq<WT, Out, 4, NW, S16><<<grid, 64 * NW, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd,
-                                                          part);
+  } else if constexpr (kq_tm_max<WT>() >= 2) {  // (not instantiated where it cannot be chosen)
+    if (f.tm == 2) {
+      k_mmq_kq<WT, Out, 2, 4, S16><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
+    } else if constexpr (kq_tm_max<WT>() >= 4) {
+      k_mmq_kq<WT, Out, 4, 4, S16><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
+    }
   }
   if (part) split_sum<Out>(part, splits, ncols_y, nrows_x, d, ldd, nullptr, s);
 }

@@ -4,7 +4,7 @@
 // Nothing here calls hipMalloc, hipFree or an allocating library routine.
 //
 // The array is `scratch`, kScratchBytes per device: kActBytes for the quantized activations, then kFixupBytes for
-// the split-K planes (the reference's tmp_fixup size for 256 compute units, fast_mmq.rs:442-444).  Each device holds
+// the split-K planes (qmm_fixup_nsm's largest, as the host layer's workspace).  Each device holds
 // its own copy until the process ends; its device address is looked up once per device, on the first call made
 // with that device current, and only that address is handed to kernels.  Every call on a device shares that
 // device's array, so calls that overlap on one device (two host threads, two streams) race; every byte a call reads
@@ -16,7 +16,7 @@
 
 namespace {
 constexpr size_t kActBytes = (size_t)16 << 20;
-constexpr size_t kFixupBytes = (size_t)16 << 20;
+constexpr size_t kFixupBytes = (size_t)QMM_MAX_FIXUP_BYTES;
 constexpr size_t kScratchBytes = kActBytes + kFixupBytes;
 constexpr int kMaxDevices = 64;
 }  // namespace
@@ -173,10 +173,11 @@ int forward(const void *w, int wtype, int64_t n, int64_t k, const void *xs, int 
    : prefill_q8k(wtype) ? launch_mmq_quantize_q8k
                         : launch_mmq_quantize_q8_1_DS4)(xs, nullptr, ptr, in_dtype, k, k, k * rows, k * rows, kp, rows, 1,
                                                         1, stream);
-  // the fixup region holds nsm * 128 * 128 f32 for nsm up to 256 (MI355X has 256 compute units); a device with more
-  // would split K less than the host layer does, and its output would then differ from QMatMul::forward's in the f32
-  // summation order
-  const int nsm = qmm_device_cus() < (int)(kFixupBytes / 65536) ? qmm_device_cus() : (int)(kFixupBytes / 65536);
+  // the fixup region holds nsm * 128 * 128 f32 for nsm up to 1024, as qmm_fixup_nsm asks at most (a device with more
+  // compute units would split K less than the host layer does, and its output would then differ from QMatMul::forward's
+  // in the f32 summation order)
+  const int want = qmm_fixup_nsm(qmm_device_cus(), wtype, n, k, rows);
+  const int nsm = want < (int)(kFixupBytes / 65536) ? want : (int)(kFixupBytes / 65536);
   mm(ptr + kActBytes, w, ptr, ys, k, n, rows, k / (int64_t)qmm_block_size(wtype), n, 0, nsm, 160 * 1024, 64, in_dtype,
      stream);
   return 0;

@@ -227,6 +227,41 @@ struct wq5k {
   }
 };
 
+// Q5_K in two planes: sc * q5 in [0, 1953] split as Q6_K's (split256), for the kernel that keeps a superblock's planes in
+// registers
+struct wq5k2 {
+  static constexpr int kBytes = 176;
+  static constexpr int kPlanes = 2;
+  static constexpr int kShift = 8;
+  static constexpr bool kMin = true;
+  static __device__ __forceinline__ int chunk(int j, int g) { return 2 * j + g; }
+  typedef wq5k::Raw Raw;
+  typedef wq5k::Prep Prep;
+  template <int PS>
+  static __device__ __forceinline__ void load_lds(const uint8_t *p, uint32_t off, int g, Raw &r) {
+    wq5k::load_lds<PS>(p, off, g, r);
+  }
+  template <bool S16 = false>
+  static __device__ __forceinline__ void prepare(const Raw &r, int g, Prep &p) {
+    wq5k::prepare<S16>(r, g, p);
+  }
+  static __device__ __forceinline__ void planes(const Raw &r, const Prep &, int j, v4i &b1, v4i &b2) {
+    wq4k::Raw h;
+    h.hdr = r.hdr;
+    const short sc = (short)wq4k::scale(h, j);
+    const s2 sc2 = {sc, sc};
+    const u32x4 q = r.q[j >> 1];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t nib = ((j & 1) ? q[i] >> 4 : q[i]) & 0x0f0f0f0fu;
+      const uint32_t hb = (j <= 4 ? r.qh[i] << (4 - j) : r.qh[i] >> (j - 4)) & 0x10101010u;
+      const uint32_t v5 = nib | hb;
+      const s2 lo = __builtin_bit_cast(s2, v5 & 0x00ff00ffu), hi = __builtin_bit_cast(s2, (v5 >> 8) & 0x00ff00ffu);
+      split256(lo * sc2 + (s2){128, 128}, hi * sc2 + (s2){128, 128}, b1, b2, i);  // w + 128
+    }
+  }
+};
+
 // Q6_K: per lane, per superblock: ql[64h + 32p + 16g ..+16], qh[32h + 16g ..+16] (h, p in {0,1}), the 8 scales
 // sc[2j + g] and d.  Chunk j (32 values 32j..32j+31) covers h = j / 4, q = j % 4, l = 16g + (0..15).
 struct wq6k {

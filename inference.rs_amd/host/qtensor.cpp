@@ -431,7 +431,7 @@ void QMatMul::forward(const void *xs, GgmlDType in_dtype, int64_t rows, void *ys
     }
   } else {
     const int64_t kp = pad_to(k, 256);
-    const int nsm = device_cus(w.device().ordinal);
+    const int nsm = qmm_fixup_nsm(device_cus(w.device().ordinal), (int)t, n, k, rows);
     Carver c;
     const size_t o_y = c.add((size_t)(rows * kp / 256 * prefill_tile_bytes_per_256(t)));
     const size_t o_fix = c.add(fixup_bytes(nsm));
@@ -458,7 +458,7 @@ void QMatMul::down_from_glu(const float *gate, const float *up, int64_t rows, in
   if (k % (int64_t)block_size(t) != 0) throw Error("QMatMul::down_from_glu: K is not a multiple of the block size");
   hip_check(hipSetDevice(w.device().ordinal), "hipSetDevice");
   const int64_t kp = pad_to(k, 256);
-  const int nsm = device_cus(w.device().ordinal);
+  const int nsm = qmm_fixup_nsm(device_cus(w.device().ordinal), (int)t, n, k, rows);
   Carver c;
   const size_t o_y = c.add((size_t)(rows * kp / 256 * prefill_tile_bytes_per_256(t)));
   const size_t o_fix = c.add(fixup_bytes(nsm));
@@ -510,7 +510,7 @@ void fused_ffn(const QMatMul &gate, const QMatMul &up, const QMatMul &down, cons
   }
   // prefill: one tile-layout quantization read by both matmuls, then down_from_glu on their f32 outputs
   const int64_t kp = pad_to(hidden, 256);
-  const int nsm = device_cus(ordinal);
+  const int nsm = qmm_fixup_nsm(device_cus(ordinal), (int)t, inter, hidden, rows);
   Carver c;
   const size_t o_y = c.add((size_t)(rows * kp / 256 * prefill_tile_bytes_per_256(t)));
   const size_t o_fix = c.add(fixup_bytes(nsm));

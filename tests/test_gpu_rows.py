@@ -112,3 +112,54 @@ def test_grouped_glu(gtype, counts):
         assert_parity(out.cpu().numpy(), want, what=f"grouped glu {gtype} {counts}")
     assert fn(*args, e, 9, qmm._stream()) == -1 and qmm.last_error()
     qmm.lib().qmm_clear_error()
+
+
+# The wide prefill tiles (256 weight rows x 64 or 128 activation rows): ragged in both, an odd number of superblocks, Q6_K
+# 2 bytes past a dword; sizes at which the dispatch's model takes them (several rounds of the other forms' tiles)
+WIDE = [(O.Q4K, 14113, 1280, 333, True), (O.Q4K, 14113, 1280, 333, False), (O.Q5K, 14113, 1280, 333, True),
+        (O.Q5K, 9999, 768, 260, False), (O.Q6K, 14113, 1280, 333, False), (O.Q6K, 14113, 1280, 61, False),
+        (O.IQ4XS, 14113, 1280, 333, False)]
+
+
+@pytest.mark.parametrize("gtype,n,k,m,q8k", WIDE)
+def test_wide_prefill_tiles(gtype, n, k, m, q8k):
+    rng = np.random.default_rng(7400 + m + k)
+    if gtype == O.IQ4XS:
+        wq = rng.integers(0, 256, n * k // 256 * 136, dtype=np.uint8)
+        wq.reshape(-1, 136)[:, :2] = (rng.uniform(0.5, 1.5, n * k // 256) * 0.002).astype(np.float16).view(
+            np.uint8).reshape(-1, 2)
+    else:
+        wq = O.quantize(gtype, weights(rng, n, k))
+    wd = dev(wq, 2 if gtype == O.Q6K else 0)
+    x = acts(rng, m, k)
+    x[m - 1] = 0.0
+    want = O.matmul(gtype, x, wq, n)
+    xd = torch.from_numpy(x).cuda()
+    got = qmm.qmatmul_prefill(gtype, wd, xd, n, q8k=q8k)
+    assert_parity(got.cpu().numpy(), want, what=f"wide {gtype} n={n} k={k} m={m}")
+    half = qmm.qmatmul_prefill(gtype, wd, xd, n, out_dtype=torch.bfloat16, q8k=q8k)
+    assert torch.equal(half.view(torch.int16), got.to(torch.bfloat16).view(torch.int16))
+
+
+@pytest.mark.parametrize("gtype,n,k,m", [(O.Q6K, 4001, 7168, 300), (O.Q5K, 1000, 7168, 500)])
+def test_wide_prefill_split_k(gtype, n, k, m):
+    """Wide tiles over more planes than the reference's fixup buffer holds, through QMatMul::forward, twice: the same bits
+    whichever split finishes first."""
+    import ctypes
+    rng = np.random.default_rng(7500 + m)
+    wq = O.quantize(gtype, weights(rng, n, k))
+    x = acts(rng, m, k)
+    H = qmm.host()
+    h = ctypes.c_void_p()
+    assert H.qmm_qtensor_from_data(gtype, wq.ctypes.data, wq.size, 1, n, k, 0, ctypes.byref(h)) == 0
+    try:
+        xd = torch.from_numpy(x).cuda()
+        outs = [torch.full((m, n), float("nan"), device="cuda") for _ in range(2)]
+        for o in outs:
+            assert H.qmm_qmatmul_forward(h, xd.data_ptr(), 0, m, o.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream) == 0, H.qmm_host_last_error()
+        torch.cuda.synchronize()
+    finally:
+        H.qmm_qtensor_free(h)
+    assert torch.equal(outs[0], outs[1])
+    assert_parity(outs[0].cpu().numpy(), O.matmul(gtype, x, wq, n), what=f"split wide {gtype} n={n} k={k} m={m}")
