@@ -257,6 +257,12 @@ void fused_glu(const void *vx_gate, const void *vx_up, const void *vy, void *dst
   }
   if (b == 0 || nrows_x == 0) return;
   hipStream_t s = (hipStream_t)stream;
+  if constexpr (F == kActQ8_0) {
+    if (b >= qmm_skinny_b32_min_rows_glu(nrows_x) &&
+        qmm_skinny_b32(T, out_type_of((const Out *)nullptr), vx_gate, vx_up, vy, dst, ncols_x, nrows_x, stride_col_y,
+                       stride_col_dst, b, activation, s))
+      return;
+  }
   if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
     if (b >= qmm_skinny_min_rows(ncols_x) &&
         qmm_skinny_glu(T, out_type_of((const Out *)nullptr), vx_gate, vx_up, vy, dst, ncols_x, nrows_x, stride_col_y,
@@ -279,15 +285,17 @@ void fused_qkv(const void *vx_q, const void *vx_k, const void *vx_v, const void 
   if (!check_weights<T, F>(who, ncols_x, stride_col_y, b, {vx_q, vx_k, vx_v}, {nrows_q, nrows_k, nrows_v})) return;
   if (b == 0 || nrows_q + nrows_k + nrows_v == 0) return;
   hipStream_t s = (hipStream_t)stream;
-  if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
-    if (b >= qmm_skinny_min_rows(ncols_x)) {
+  if constexpr (F == kActQ8_0 || T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
+    if (b >= (F == kActQ8_0 ? QMM_SKINNY_B32_MIN_ROWS_QKV : qmm_skinny_min_rows(ncols_x))) {
       const int ot = out_type_of((const Out *)nullptr);
       const void *w[3] = {vx_q, vx_k, vx_v};
       void *d[3] = {q_dst, k_dst, v_dst};
       const int n[3] = {nrows_q, nrows_k, nrows_v};
       bool ok = true;
       for (int i = 0; i < 3 && ok; i++)
-        if (n[i] > 0) ok = qmm_skinny_decode(T, ot, w[i], vy, d[i], ncols_x, n[i], stride_col_y, n[i], b, s);
+        if (n[i] > 0)
+          ok = F == kActQ8_0 ? qmm_skinny_b32(T, ot, w[i], nullptr, vy, d[i], ncols_x, n[i], stride_col_y, n[i], b, 0, s)
+                             : qmm_skinny_decode(T, ot, w[i], vy, d[i], ncols_x, n[i], stride_col_y, n[i], b, s);
       if (ok) return;
     }
   }

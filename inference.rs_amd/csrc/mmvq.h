@@ -1043,8 +1043,14 @@ void plain_t(const void *vx, const void *vy, void *dst, int ncols_x, int nrows_x
   hipStream_t s = (hipStream_t)stream;
   const uint8_t *x = (const uint8_t *)vx, *y = (const uint8_t *)vy;
   typename Out::T *d = (typename Out::T *)dst;
-  if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q6K) {
-    if (b >= qmm_skinny_min_rows(ncols_x) &&
+  if constexpr (F == kActQ8_0) {
+    if (b >= qmm_skinny_b32_min_rows(nrows_x, ncols_x) &&
+        qmm_skinny_b32(T, out_type_of((const Out *)nullptr), vx, nullptr, vy, dst, ncols_x, nrows_x, stride_col_y,
+                       stride_col_dst, b, 0, s))
+      return;
+  }
+  if constexpr (T == QMM_TYPE_Q4K || T == QMM_TYPE_Q5K || T == QMM_TYPE_Q6K) {
+    if (b >= (T == QMM_TYPE_Q5K ? qmm_skinny_b32_min_rows(nrows_x, ncols_x) : qmm_skinny_min_rows(ncols_x)) &&
         qmm_skinny_decode(T, out_type_of((const Out *)nullptr), vx, vy, dst, ncols_x, nrows_x, stride_col_y,
                           stride_col_dst, b, s))
       return;

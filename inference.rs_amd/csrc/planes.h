@@ -465,6 +465,8 @@ __device__ __forceinline__ v4f mfma16_f16(v4h a, v4h b, v4f c) {
 // chunks of nibbles.  The min term: lane group kg carries sub-blocks 4p + 2(kg/2) + {0, 1} with p = kg % 2, the ones
 // whose activation sums it can form from its own A fragments and its partner's (lane ^ 16).
 struct wq4k16 {
+  static constexpr bool kB32 = false;
+  static constexpr int kRows = 32;  // activation rows the decode entries take
   static constexpr int kBytes = 144;
   static constexpr int kPieces = 9;  // 16-byte pieces of a superblock (of its window) in LDS
   static constexpr int kShift = 3;
@@ -519,6 +521,8 @@ struct wq4k16 {
 // Q6_K: step t takes values 64t + 16kg + (0..15): low (t even) or high (t odd) nibbles of ql[64(t/2) + 16kg ..],
 // the 2-bit fields 2q, q = 2(t%2) + kg/2, of qh[32(t/2) + 16(kg%2) ..], scale sc[4t + kg].
 struct wq6k16 {
+  static constexpr bool kB32 = false;
+  static constexpr int kRows = 32;  // activation rows the decode entries take
   static constexpr int kBytes = 210;
   static constexpr int kPieces = 14;
   static constexpr int kShift = 8;  // split256
@@ -584,5 +588,103 @@ struct wq6k16 {
       const s2 hi = __builtin_bit_cast(s2, (v6 >> 8) & 0x00ff00ffu);
       split256(lo * sc2 + c2, hi * sc2 + c2, b1, b2, i);  // w + 128
     }
+  }
+};
+
+// Q5_K: Q4_K's steps with the fifth bits (planes.h wq5k2): sc * q5 split as Q6_K's.  Byte 16 (kg % 2) + l of qh holds the
+// fifth bits of value l of this lane's half of every sub-block, bit j of it sub-block j's.
+struct wq5k16 {
+  static constexpr bool kB32 = false;
+  static constexpr int kRows = 16;  // activation rows the decode entries take
+  static constexpr int kBytes = 176;
+  static constexpr int kPieces = 11;
+  static constexpr int kShift = 8;  // split256
+  static constexpr bool kMin = true;
+  struct Raw {
+    u32x4 hdr, qh, q[2];
+  };
+  static __device__ __forceinline__ uint32_t act_offset(int t, int kg) { return wq4k16::act_offset(t, kg); }
+  static __device__ __forceinline__ void load_lds(const uint8_t *p, uint32_t, int kg, Raw &r) {
+    r.hdr = *(const u32x4 *)p;
+    r.qh = *(const u32x4 *)(p + 16 + 16 * (kg & 1));
+    r.q[0] = *(const u32x4 *)(p + 48 + 16 * kg);
+    r.q[1] = *(const u32x4 *)(p + 112 + 16 * kg);
+  }
+  struct Prep {
+    wq4k16::Prep k;
+    float d, dmin;
+    v4h bmin;
+    uint32_t qh[4];  // shifted: bit 4p + h is sub-block 4p + 2 (kg / 2) + h's
+  };
+  static __device__ __forceinline__ void prepare(const Raw &r, int kg, Prep &p) {
+    wq4k16::Raw h;
+    h.hdr = r.hdr;
+    wq4k16::prepare(h, kg, p.k);
+    p.d = p.k.d;
+    p.dmin = p.k.dmin;
+    p.bmin = p.k.bmin;
+    const uint32_t sft = 2 * (kg >> 1);
+#pragma unroll
+    for (int i = 0; i < 4; i++) p.qh[i] = r.qh[i] >> sft;
+  }
+  static __device__ __forceinline__ void planes(const Raw &r, const Prep &p, int t, v4i &b1, v4i &b2, int) {
+    const int bit = 4 * (t >> 1) + (t & 1);
+    const short sc = (short)(8 * p.k.sh[t] + p.k.sl[t]);
+    const s2 sc2 = {sc, sc};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t nib = ((t & 1) ? r.q[t >> 1][i] >> 4 : r.q[t >> 1][i]) & 0x0f0f0f0fu;
+      const uint32_t v5 = nib | ((bit <= 4 ? p.qh[i] << (4 - bit) : p.qh[i] >> (bit - 4)) & 0x10101010u);
+      const s2 lo = __builtin_bit_cast(s2, v5 & 0x00ff00ffu), hi = __builtin_bit_cast(s2, (v5 >> 8) & 0x00ff00ffu);
+      split256(lo * sc2 + (s2){128, 128}, hi * sc2 + (s2){128, 128}, b1, b2, i);  // w + 128
+    }
+  }
+};
+
+// ------------------------------------------------------------------------------------------ 32-value blocks, 16x16x32
+
+// Operands of v_mfma_i32_16x16x32_i8, one 32-value block a step: lane (kg, r) holds values 4kg .. 4kg + 3 and 16 + 4kg ..
+// 19 + 4kg of row r's block as two dwords, on both sides.  The weight bytes are 2^kUp times the values, so that the 4- and
+// 5-bit ones need no sign extension: 16 (q - 8) is the nibble at the top of its byte with the byte's top bit flipped, 8 (q
+// - 16) the five bits likewise; the scale makes up for it (an exact power of two).
+__device__ __forceinline__ v4i mfma16x32_i8(u32x2 a, u32x2 b) {
+  return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, a), __builtin_bit_cast(long, b), (v4i){}, 0, 0, 0);
+}
+// the dword at byte `o` of the dword-aligned LDS row p (o % 4 is 0 or 2)
+__device__ __forceinline__ uint32_t lds_dw(const uint8_t *p, int o, int kg) {
+  const uint32_t *q = (const uint32_t *)(p + (o & ~3)) + kg;
+  return o % 4 == 0 ? q[0] : __builtin_amdgcn_alignbyte(q[1], q[0], 2);
+}
+// block j of the superblock at p: its two operand dwords and its f16 scale
+struct wb16_q8_0 {
+  static constexpr bool kB32 = true;
+  static constexpr int kRows = 16;  // activation rows the decode entries take
+  static constexpr int kBytes = 272, kPieces = 17, kUp = 0;  // a superblock of eight 34-byte blocks
+  static __device__ __forceinline__ u32x2 block(const uint8_t *p, int j, int kg, uint32_t &d) {
+    d = *(const uint16_t *)(p + 34 * j);
+    return (u32x2){lds_dw(p, 34 * j + 2, kg), lds_dw(p, 34 * j + 18, kg)};
+  }
+};
+struct wb16_q4_0 {
+  static constexpr bool kB32 = true;
+  static constexpr int kRows = 16;  // activation rows the decode entries take
+  static constexpr int kBytes = 144, kPieces = 9, kUp = 4;
+  static __device__ __forceinline__ u32x2 block(const uint8_t *p, int j, int kg, uint32_t &d) {
+    d = *(const uint16_t *)(p + 18 * j);
+    const uint32_t q = lds_dw(p, 18 * j + 2, kg);
+    return (u32x2){((q << 4) & 0xf0f0f0f0u) ^ 0x80808080u, (q & 0xf0f0f0f0u) ^ 0x80808080u};
+  }
+};
+struct wb16_q5_0 {
+  static constexpr bool kB32 = true;
+  static constexpr int kRows = 16;  // activation rows the decode entries take
+  static constexpr int kBytes = 176, kPieces = 11, kUp = 3;
+  static __device__ __forceinline__ u32x2 block(const uint8_t *p, int j, int kg, uint32_t &d) {
+    d = *(const uint16_t *)(p + 22 * j);
+    const uint32_t qh = lds_dw(p, 22 * j + 2, 0) >> (4 * kg);  // bit v: the fifth bit of value v
+    const uint32_t q = lds_dw(p, 22 * j + 6, kg);
+    const uint32_t h0 = (((qh & 15u) * 0x00204081u) & 0x01010101u) << 7;
+    const uint32_t h1 = ((((qh >> 16) & 15u) * 0x00204081u) & 0x01010101u) << 7;
+    return (u32x2){(((q << 3) & 0x78787878u) | h0) ^ 0x80808080u, (((q >> 1) & 0x78787878u) | h1) ^ 0x80808080u};
   }
 };

@@ -11,9 +11,25 @@
 // Q6_K 1024x4096 3.1 and 5.3; two rows of wide weights Q6_K 4096x14336 17.9 and 14.4, Q4_K 8192x8192 14.3 and 11.1.
 inline int qmm_skinny_min_rows(int64_t k) { return k >= 8192 ? 2 : 3; }
 
-// Decode-layout activations (b rows of Q8_K blocks, stride_col_y blocks apart) against Q4_K / Q6_K weights;
+// The same for Q8_0 / Q4_0 / Q5_0 and Q5_K weights of n rows.  The kernel's time does not grow with the rows, the matvec's
+// does; narrow weights leave the kernel with few workgroups.  MI355X, us, matvec and this kernel, Q8_0 unless said
+// otherwise: 1024x4096 8 rows 5.2 / 5.6, 16 rows 9.8 / 5.6; 2048x4096 5 rows 5.6 / 6.0, 6 rows 6.5 / 6.0; 4096x4096 3 rows
+// 7.0 / 7.3, 4 rows 8.3 / 7.3; 4096x14336 3 rows 21.8 / 15.5; 14336x4096 3 rows 16.5 / 14.2, 16 rows 60.6 / 14.7, Q5_K 3
+// rows 13.8 / 12.7, Q4_0 12.1 / 10.2, Q5_0 13.3 / 12.3; 2 rows 14.0 / 14.9.
+inline int qmm_skinny_b32_min_rows(int64_t n, int64_t k) {
+  return n < 2048 ? 9 : n < 4096 ? 6 : n < 8192 && k < 8192 ? 4 : 3;
+}
+// Fused forms of the 32-value types.  Gate and up, 2 x n rows: 2 x 2048x2048 4 rows 5.7 / 5.6, 6 rows 9.8 / 5.6; 2 x
+// 14336x4096 2 rows 23.0 / 23.8, 3 rows 29.7 / 23.6, 16 rows 115 / 25.  Q, K and V are three launches here and one matvec:
+// (2048 + 2 x 512)x2048 6 rows 10.4 / 12.0, 8 rows 11.9 / 11.9; (4096 + 2 x 1024)x4096 4 rows 14.4 / 18.6, 8 rows 26.9 /
+// 18.7.
+inline int qmm_skinny_b32_min_rows_glu(int64_t n) { return n < 4096 ? 5 : 3; }
+constexpr int QMM_SKINNY_B32_MIN_ROWS_QKV = 8;
+
+// Decode-layout activations (b rows of Q8_K blocks, stride_col_y blocks apart) against Q4_K / Q5_K / Q6_K weights;
 // dst[j * stride_col_dst + row] of element type out_type (QMM_TYPE_F32 / F16 / BF16).  Returns false, launching
-// nothing, for a case it does not serve (other weight types, b outside 1..32, K not a multiple of 256).
+// nothing, for a case it does not serve (other weight types, b outside 1..32 (Q5_K 1..16),
+// K not a multiple of 256).
 bool qmm_skinny_decode(int type, int out_type, const void *vx, const void *vy, void *dst, int ncols_x, int nrows_x,
                        int stride_col_y, int stride_col_dst, int b, hipStream_t s);
 
@@ -21,6 +37,11 @@ bool qmm_skinny_decode(int type, int out_type, const void *vx, const void *vy, v
 bool qmm_skinny_glu(int type, int out_type, const void *vx_gate, const void *vx_up, const void *vy, void *dst,
                     int ncols_x, int nrows_x, int stride_col_y, int stride_col_dst, int b, int activation,
                     hipStream_t s);
+
+// The same for Q8_0 / Q4_0 / Q5_0 weights against rows of Q8_0 blocks (stride_col_y blocks apart), b in 1..16; vx2: the
+// up weights of the GLU form, null for a plain product.
+bool qmm_skinny_b32(int type, int out_type, const void *vx, const void *vx2, const void *vy, void *dst, int ncols_x,
+                    int nrows_x, int stride_col_y, int stride_col_dst, int b, int activation, hipStream_t s);
 
 // The same over the tensor-core entries' activation layout (rows of ncols_x / 256 blocks {f32 d; int8 qs[256]},
 // units.h), for launch_mmvq_tc_gguf_<t>_*_plain.

@@ -1,4 +1,4 @@
-// Few-row matmul for K-quant weights on int8 MFMA: up to 32 activation rows against a weight matrix streamed once from
+// Few-row matmul on int8 MFMA: up to 32 activation rows (16 for Q5_K and the 32-value types) against a weight matrix streamed once from
 // HBM.  Serves the decode matvec from a few rows on (the reference's tensor-core matvec, mmvq_tc_k.cuh,
 // fast_mmvq.rs:1897-2126, and its plain launcher at b <= 8), its fused GLU form, and the expert-grouped matmul when the
 // experts receive few rows each.
@@ -17,7 +17,11 @@
 //
 // Each wave's lane (kg, r) builds the two int8 weight planes of row r (planes.h) as the MFMA B column, with activation
 // row r as the A row; one 16x16x64 MFMA per plane per 64 values, the Q4_K min term through one f16 MFMA per superblock,
-// and the per-superblock f32 scaling of the reference (k_quants.rs:1848-1928, 2518-2575).
+// and the per-superblock f32 scaling of the reference (k_quants.rs:1848-1928, 2145-2232, 2518-2575).  Weights of 32-value
+// blocks (Q8_0, Q4_0, Q5_0) against Q8_0 activations stage superblocks of eight blocks the same way and take one 16x16x32
+// MFMA a block, whose sums are scaled by both blocks' scales (432-449, 615-637, 982-999): 4 conversions, 4 products and 4
+// fused adds a lane and block, which the loads cover.  11008x4096 Q8_0 at 5 / 16 rows 12.5 / 13.1 us, 3.8 TB/s (the matvec
+// 21 / 53); 32768x4096 27.1 / 28.4, 5.3 TB/s (44 / 101).
 #include "common.h"
 #include "inferencequant.h"
 #include "planes.h"
@@ -59,12 +63,38 @@ constexpr uint32_t kNowhere = 0x80000000u;  // past every resource's end: reads 
 template <class WT, int NW, int TC, int MT, int D>
 struct RowsLds {
   static constexpr int kUnit = 256 * WT::kPieces;            // a unit's window: 16 rows x kPieces 16-byte pieces
-  static constexpr int kAct = 256 * 16 * MT + 4 * 16 * MT;   // a superblock's activations: rows (chunk c of row m at
-                                                             // c ^ (m % 16)), then the scales
+  // a superblock's activations: 16 MT rows of 256 values (chunk c of row m at c ^ (m % 16)), then their scales; for the
+  // 32-value types 16 rows of eight 34-byte Q8_0 blocks
+  static constexpr int kAct = WT::kB32 ? 272 * 16 * MT : 256 * 16 * MT + 4 * 16 * MT;
   static constexpr int kWave = kAct + D * kUnit;
   static constexpr int kSums = NW * TC * MT * 1024;          // the partial sums, in the same memory afterwards
   static constexpr int kBytes = NW * kWave > kSums ? NW * kWave : kSums;
 };
+
+// A superblock's activations in registers: operand rows, f32 scales of the four output rows, the Q4_K / Q5_K min operand
+template <bool B32, int MT>
+struct ActRegs {
+  struct T {
+    v4i q[MT][4];
+    v4f d[MT];
+    v4h m[MT];
+  };
+};
+template <int MT>
+struct ActRegs<true, MT> {
+  static_assert(MT == 1, "32-value types take 16 rows");
+  struct T {
+    u32x2 q[8];  // per block
+    v4f d[8];
+  };
+};
+template <class WT>
+constexpr bool has_min() {
+  if constexpr (WT::kB32)
+    return false;
+  else
+    return WT::kMin;
+}
 
 // One pass: the workgroup's 16 TN weight rows from n0 against activation rows [m0, m0 + mr), mr <= 16 MT.
 // MT: 16-row activation tiles (1 or 2).  GLU: tiles [0, TC / 2) are gate rows (W), [TC / 2, TC) the up rows (W2) at the
@@ -78,7 +108,7 @@ __device__ __forceinline__ void rows_pass(uint8_t *lds, const uint8_t *__restric
   constexpr int MR = 16 * MT;            // activation rows
   constexpr int TN = GLU ? TC / 2 : TC;  // tiles of output columns
   constexpr int P = WT::kPieces, UB = L::kUnit;
-  constexpr int LW = (16 * P + 63) / 64, LA = MR / 4 + 1;  // DMA loads of a unit and of a superblock's activations
+  constexpr int LW = (16 * P + 63) / 64, LA = WT::kB32 ? (17 * MR + 63) / 64 : MR / 4 + 1;  // DMA loads of a unit and of a superblock's activations
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, kg = lane >> 4,
             r = lane & 15;
@@ -119,20 +149,28 @@ __device__ __forceinline__ void rows_pass(uint8_t *lds, const uint8_t *__restric
 
   // wave w takes superblocks w, w + NW, ...: what the waves have in flight at a time is one run of each row
   const int s0 = wave, s1 = nsb;
-  uint32_t aoff[MR / 4];
+  uint32_t aoff[LA];
 #pragma unroll
-  for (int i = 0; i < MR / 4; i++) {
-    const int row = 4 * i + kg, c = r ^ (row & 15);
-    aoff[i] = row < mr ? ap.q0 + (uint32_t)(m0 + row) * ap.qrow + 16 * c : kNowhere;
+  for (int i = 0; i < LA; i++) {
+    // row and 16-byte chunk of this lane's i-th load (the last one of the K-quants: the scales, dwords)
+    const int C = 64 * i + lane, row = WT::kB32 ? C / 17 : i < MR / 4 ? C / 16 : lane;
+    const uint32_t in_row = WT::kB32 ? 16 * (C - 17 * row) : i < MR / 4 ? 16 * (r ^ (row & 15)) : 0;
+    aoff[i] = row < mr ? (WT::kB32 || i < MR / 4 ? ap.q0 + (uint32_t)(m0 + row) * ap.qrow
+                                                : ap.d0 + (uint32_t)(m0 + row) * ap.drow) + in_row
+                       : kNowhere;
   }
-  const uint32_t doff = lane < mr ? ap.d0 + (uint32_t)(m0 + lane) * ap.drow : kNowhere;
   auto issue_a = [&](int sb, bool skip) {
     const rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)ap.base, (short)0, skip ? 0 : (int)ap.bytes, 0x00020000);
     const uint32_t oq = (uint32_t)sb * ap.qsb, od = (uint32_t)sb * ap.dsb;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < MR / 4; i++) dma16(ra, abuf + 1024 * i, aoff[i], oq);
-    if (lane < MR) dma4(ra, abuf + 256 * MR, doff, od);
+    for (int i = 0; i < LA; i++) {
+      if (!WT::kB32 && i == MR / 4) {
+        if (lane < MR) dma4(ra, abuf + 256 * MR, aoff[i], od);
+      } else if (!WT::kB32 || 64 * i + 64 <= 17 * MR || lane < 17 * MR - 64 * i) {
+        dma16(ra, abuf + 1024 * i, aoff[i], oq);
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -150,19 +188,29 @@ __device__ __forceinline__ void rows_pass(uint8_t *lds, const uint8_t *__restric
     for (int sb = s0; sb < s1; sb += NW) {
       // the activations of sb have landed once at most the weight loads issued after them are outstanding
       wait_vm<(TC < D ? TC : D) * LW>();
-      v4i aq[MT][4];
-      v4f dy[MT];
-      v4h am[MT];
+      typename ActRegs<WT::kB32, MT>::T act;
+      if constexpr (WT::kB32) {
 #pragma unroll
-      for (int x = 0; x < MT; x++) {
+        for (int j = 0; j < 8; j++) {
+          act.q[j] = (u32x2){lds_dw(abuf + 272 * r, 34 * j + 2, kg), lds_dw(abuf + 272 * r, 34 * j + 18, kg)};
 #pragma unroll
-        for (int t = 0; t < 4; t++)
-          aq[x][t] = *(const v4i *)(abuf + 256 * (16 * x + r) + 16 * ((WT::act_offset(t, kg) / 16) ^ r));
-        dy[x] = *(const v4f *)(abuf + 256 * MR + 4 * (16 * x + 4 * kg));
+          for (int i = 0; i < 4; i++) {
+            const _Float16 h = __builtin_bit_cast(_Float16, *(const uint16_t *)(abuf + 272 * (4 * kg + i) + 34 * j));
+            act.d[j][i] = (float)h;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int x = 0; x < MT; x++) {
+#pragma unroll
+          for (int t = 0; t < 4; t++)
+            act.q[x][t] = *(const v4i *)(abuf + 256 * (16 * x + r) + 16 * ((WT::act_offset(t, kg) / 16) ^ r));
+          act.d[x] = *(const v4f *)(abuf + 256 * MR + 4 * (16 * x + 4 * kg));
+        }
       }
       wait_lds();
       issue_a(sb + NW, sb + NW >= s1);
-      if (WT::kMin) {
+      if constexpr (has_min<WT>()) {
         // the 32-value sums of the two sub-blocks this lane's min operand carries: its own halves plus its
         // partner's (lane ^ 16), split as planes.h min_frag does
 #pragma unroll
@@ -172,14 +220,14 @@ __device__ __forceinline__ void rows_pass(uint8_t *lds, const uint8_t *__restric
           for (int t = 0; t < 4; t++) {
             int acc = 0;
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc = sdot4(aq[x][t][i], 0x01010101, acc);
+            for (int i = 0; i < 4; i++) acc = sdot4(act.q[x][t][i], 0x01010101, acc);
             s[t] = (uint32_t)acc;
           }
           swap_lane_rows(s[0], s[2]);
           swap_lane_rows(s[1], s[3]);
           uint32_t hp, lp;
           s32_split(((s[0] + s[2]) & 0xffffu) | ((s[1] + s[3]) << 16), hp, lp);
-          am[x] = __builtin_bit_cast(v4h, (u32x2){hp, lp});
+          act.m[x] = __builtin_bit_cast(v4h, (u32x2){hp, lp});
         }
       }
 #pragma unroll
@@ -191,43 +239,59 @@ __device__ __forceinline__ void rows_pass(uint8_t *lds, const uint8_t *__restric
         else
           wait_vm<(D - 1) * LW>();
         uint8_t *const wslot = wbuf + UB * slot;
-        typename WT::Raw raw;
-        const uint32_t o = (uint32_t)(r * w_row_bytes) + (uint32_t)sb * WT::kBytes + (GLU && t >= TN ? dl2 : dl) +
-                           (WT::kBytes % 4 ? (uint32_t)(GLU && t >= TN ? t - TN : t) * tile_bytes : 0u);
-        WT::load_lds(wslot + 16 * P * r, o & 3, kg, raw);
-        wait_lds();
-        {
+        auto next_unit = [&]() {  // the unit's bytes are in registers: its slot is free
           const int tn = (t + D) % TC, sn = sb + (t + D) / TC * NW;
+          wait_lds();
           issue_w(tn, sn, wslot, sn >= s1);
-        }
-        slot = slot + 1 == D ? 0 : slot + 1;
-        typename WT::Prep p;
-        WT::prepare(raw, kg, p);
-        v4i acc1[MT], acc2[MT];
+        };
+        if constexpr (WT::kB32) {
+          u32x2 wv[8];
+          uint32_t wd[8];
 #pragma unroll
-        for (int x = 0; x < MT; x++) acc1[x] = acc2[x] = (v4i){};
+          for (int j = 0; j < 8; j++) wv[j] = WT::block(wslot + 16 * P * r, j, kg, wd[j]);
+          next_unit();
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          v4i b1, b2;
-          WT::planes(raw, p, q, b1, b2, kg);
+          for (int j = 0; j < 8; j++) {
+            const v4i iv = mfma16x32_i8(act.q[j], wv[j]);
+            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)wd[j]) * (1.0f / (1 << WT::kUp));
+#pragma unroll
+            for (int i = 0; i < 4; i++) fa[t][0][i] = __builtin_fmaf(act.d[j][i], d * (float)iv[i], fa[t][0][i]);
+          }
+        } else {
+          typename WT::Raw raw;
+          const uint32_t o = (uint32_t)(r * w_row_bytes) + (uint32_t)sb * WT::kBytes + (GLU && t >= TN ? dl2 : dl) +
+                             (WT::kBytes % 4 ? (uint32_t)(GLU && t >= TN ? t - TN : t) * tile_bytes : 0u);
+          WT::load_lds(wslot + 16 * P * r, o & 3, kg, raw);
+          next_unit();
+          typename WT::Prep p;
+          WT::prepare(raw, kg, p);
+          v4i acc1[MT], acc2[MT];
+#pragma unroll
+          for (int x = 0; x < MT; x++) acc1[x] = acc2[x] = (v4i){};
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            v4i b1, b2;
+            WT::planes(raw, p, q, b1, b2, kg);
+#pragma unroll
+            for (int x = 0; x < MT; x++) {
+              acc1[x] = mfma16_i8(act.q[x][q], b1, acc1[x]);
+              acc2[x] = mfma16_i8(act.q[x][q], b2, acc2[x]);
+            }
+          }
 #pragma unroll
           for (int x = 0; x < MT; x++) {
-            acc1[x] = mfma16_i8(aq[x][q], b1, acc1[x]);
-            acc2[x] = mfma16_i8(aq[x][q], b2, acc2[x]);
+            v4f fmin = (v4f){};
+            if (WT::kMin) fmin = mfma16_f16(act.m[x], p.bmin, fmin);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const int iv = (acc1[x][i] << WT::kShift) + acc2[x][i];
+              float v = p.d * (float)iv;
+              if (WT::kMin) v = __builtin_fmaf(-p.dmin, fmin[i], v);
+              fa[t][x][i] = __builtin_fmaf(act.d[x][i], v, fa[t][x][i]);
+            }
           }
         }
-#pragma unroll
-        for (int x = 0; x < MT; x++) {
-          v4f fmin = (v4f){};
-          if (WT::kMin) fmin = mfma16_f16(am[x], p.bmin, fmin);
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const int iv = (acc1[x][i] << WT::kShift) + acc2[x][i];
-            float v = p.d * (float)iv;
-            if (WT::kMin) v = __builtin_fmaf(-p.dmin, fmin[i], v);
-            fa[t][x][i] = __builtin_fmaf(dy[x][i], v, fa[t][x][i]);
-          }
-        }
+        slot = slot + 1 == D ? 0 : slot + 1;
         // (the sums are formed here: left alone, the compiler sinks every tile's scaling to the loop's end and keeps their
         // MFMA results in registers until then, up to 75 more)
 #pragma unroll
@@ -301,22 +365,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
   }
 }
 
-template <class WT>
-struct Wt16;
-template <>
-struct Wt16<wq4k> {
-  typedef wq4k16 T;
-};
-template <>
-struct Wt16<wq6k> {
-  typedef wq6k16 T;
-};
-
 template <class WT, class Out, int NW, int TC, int MT, bool GLU>
 void launch_k(const void *w, const void *w2, int64_t nrows, int64_t wrb, const act_rows &ap, int mrows, int64_t nsb,
               void *dst, int64_t ldd, int activation, hipStream_t s) {
   constexpr int cols = 16 * (GLU ? TC / 2 : TC);
-  k_rows<typename Wt16<WT>::T, Out, NW, TC, MT, 2, MT == 1 ? 4 : 3, GLU><<<(unsigned)qmm_ceil_div(nrows, cols), 64 * NW, 0, s>>>(
+  k_rows<WT, Out, NW, TC, MT, 2, (WT::kB32 || MT > 1 ? 3 : 4), GLU><<<(unsigned)qmm_ceil_div(nrows, cols), 64 * NW, 0, s>>>(
       (const uint8_t *)w, (const uint8_t *)w2, nrows, wrb, ap, mrows, (int)nsb, (typename Out::T *)dst, ldd, activation);
 }
 
@@ -337,6 +390,11 @@ void launch_mt(const void *w, const void *w2, int64_t nrows, int64_t wrb, const 
   //   14.7 / 15.2 / 17.3
   //   GLU 2 x 14336 (4, 4) 15.6 / 17.4 / 21.0, (4, 2) 16.7 / 19.3 / 23.3; 2 x 8960x3072 (4, 2) 10.6 / 11.8 / 14.7, (4, 4)
   //   11.5 / 12.8 / 15.9; Q6_K 2 x 11008 (4, 2) 19.1 / 20.3 / 23.9, (4, 4) 22.2 / 23.1 / 26.5
+  // and at 3 / 16 rows, K = 4096, the types that take 16 rows:
+  //   Q8_0 N = 8192 (4, 2) 9.1 / 9.5, (8, 2) 9.6 / 9.9; Q4_0 (8, 2) 7.6 / 8.0, (4, 2) 8.4 / 8.5; Q5_0 (8, 2) 9.1 / 9.4, (4, 2)
+  //   9.8 / 9.6; Q5_K (4, 2) 8.9 / 8.7, (8, 2) 9.0 / 9.4; N = 14336 Q8_0 (8, 4) 14.2 / 14.7, (4, 4) 13.9 / 14.9, (4, 6)
+  //   34 / 34, Q4_0 (8, 4) 10.4 / 10.7, (4, 4) 12.6 / 12.0; N = 32768 Q8_0 (4, 4) 27.1 / 28.4, (8, 4) 28.8 / 29.8, (4, 6)
+  //   41.5 / 42.1, Q5_K (4, 4) 22.4 / 22.8, (8, 4) 22.2 / 24.4, (4, 6) 29 / 30 (more tiles spill)
   // (the 32x32x32 and 16x16x64 kernels with register-loaded operands before this one: N = 14336 14.5 / 17.0 / 18.5, N =
   // 4096 5.5 / 6.7 / 9.3, Q6_K 4096x14336 22.9 / 26.1 / 31.4, GLU 2 x 14336 28.3 / 33.5 / 37.0)
   if (w2) {
@@ -347,9 +405,14 @@ void launch_mt(const void *w, const void *w2, int64_t nrows, int64_t wrb, const 
   } else if (tiles <= cus) {
     QMM_L(8, 1, false);
   } else if (tiles <= 2 * cus) {
-    QMM_L(4, 2, false);
+    if constexpr (WT::kB32 && WT::kBytes < 272)
+      QMM_L(8, 2, false);
+    else
+      QMM_L(4, 2, false);
   } else if (tiles <= 4 * cus) {
     QMM_L(8, 4, false);
+  } else if constexpr (WT::kB32 || WT::kRows == 16) {
+    QMM_L(4, 4, false);
   } else if (tiles <= 6 * cus) {
     QMM_L(4, 6, false);
   } else {
@@ -362,35 +425,50 @@ template <class WT, class Out>
 void launch_decode(const void *vx, const void *vx2, const act_rows &ap, void *dst, int ncols_x, int nrows_x,
                    int stride_col_dst, int b, int activation, hipStream_t s) {
   const int64_t nsb = ncols_x / 256, wrb = nsb * WT::kBytes;
-  if (b <= 16)
-    launch_mt<WT, Out, 1>(vx, vx2, nrows_x, wrb, ap, b, nsb, dst, stride_col_dst, activation, s);
-  else
-    launch_mt<WT, Out, 2>(vx, vx2, nrows_x, wrb, ap, b, nsb, dst, stride_col_dst, activation, s);
+  if constexpr (WT::kRows > 16) {
+    if (b > 16) return launch_mt<WT, Out, 2>(vx, vx2, nrows_x, wrb, ap, b, nsb, dst, stride_col_dst, activation, s);
+  }
+  launch_mt<WT, Out, 1>(vx, vx2, nrows_x, wrb, ap, b, nsb, dst, stride_col_dst, activation, s);
 }
 
-bool dispatch(int type, int out_type, const void *vx, const void *vx2, const act_rows &ap, void *dst, int ncols_x,
-              int nrows_x, int stride_col_dst, int b, int activation, hipStream_t s) {
-  if (type != QMM_TYPE_Q4K && type != QMM_TYPE_Q6K) return false;
+template <class WT>
+bool dispatch_out(int out_type, const void *vx, const void *vx2, const act_rows &ap, void *dst, int ncols_x, int nrows_x,
+                  int stride_col_dst, int b, int activation, hipStream_t s) {
   // a workgroup's rows (128 at most) are addressed with 31 bits
-  if (128 * ((int64_t)ncols_x / 256 * (int64_t)qmm_type_size(type) + 16) > 0x7ffffff0) return false;
-#define QMM_SK(WT)                                                                                                   \
-  switch (out_type) {                                                                                                \
-    case QMM_TYPE_F16:                                                                                               \
-      launch_decode<WT, out_f16>(vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);              \
-      break;                                                                                                         \
-    case QMM_TYPE_BF16:                                                                                              \
-      launch_decode<WT, out_bf16>(vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);             \
-      break;                                                                                                         \
-    default: launch_decode<WT, out_f32>(vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);       \
+  if (b > WT::kRows || 128 * ((int64_t)ncols_x / 256 * WT::kBytes + 16) > 0x7ffffff0) return false;
+  switch (out_type) {
+    case QMM_TYPE_F16:
+      launch_decode<WT, out_f16>(vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);
+      break;
+    case QMM_TYPE_BF16:
+      launch_decode<WT, out_bf16>(vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);
+      break;
+    default: launch_decode<WT, out_f32>(vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);
   }
-  if (type == QMM_TYPE_Q4K) {
-    QMM_SK(wq4k)
-  } else {
-    QMM_SK(wq6k)
-  }
-#undef QMM_SK
   return true;
 }
+
+#define QMM_SK(WT) \
+  return dispatch_out<WT>(out_type, vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s)
+bool dispatch_kq(int type, int out_type, const void *vx, const void *vx2, const act_rows &ap, void *dst, int ncols_x,
+                 int nrows_x, int stride_col_dst, int b, int activation, hipStream_t s) {
+  switch (type) {
+    case QMM_TYPE_Q4K: QMM_SK(wq4k16);
+    case QMM_TYPE_Q5K: QMM_SK(wq5k16);
+    case QMM_TYPE_Q6K: QMM_SK(wq6k16);
+    default: return false;
+  }
+}
+bool dispatch_b32(int type, int out_type, const void *vx, const void *vx2, const act_rows &ap, void *dst, int ncols_x,
+                  int nrows_x, int stride_col_dst, int b, int activation, hipStream_t s) {
+  switch (type) {
+    case QMM_TYPE_Q8_0: QMM_SK(wb16_q8_0);
+    case QMM_TYPE_Q4_0: QMM_SK(wb16_q4_0);
+    case QMM_TYPE_Q5_0: QMM_SK(wb16_q5_0);
+    default: return false;
+  }
+}
+#undef QMM_SK
 
 // Q8_1 slots (units.h): rows of 288-byte slots {f32 d; int8 qs[256]; int16 s32[8]; pad}
 bool slot_rows(const void *vy, int ncols_x, int stride_col_y, int b, act_rows &ap) {
@@ -407,7 +485,7 @@ bool qmm_skinny_decode(int type, int out_type, const void *vx, const void *vy, v
                        int stride_col_y, int stride_col_dst, int b, hipStream_t s) {
   act_rows ap;
   return slot_rows(vy, ncols_x, stride_col_y, b, ap) &&
-         dispatch(type, out_type, vx, nullptr, ap, dst, ncols_x, nrows_x, stride_col_dst, b, 0, s);
+         dispatch_kq(type, out_type, vx, nullptr, ap, dst, ncols_x, nrows_x, stride_col_dst, b, 0, s);
 }
 
 bool qmm_skinny_glu(int type, int out_type, const void *vx_gate, const void *vx_up, const void *vy, void *dst,
@@ -415,7 +493,18 @@ bool qmm_skinny_glu(int type, int out_type, const void *vx_gate, const void *vx_
                     hipStream_t s) {
   act_rows ap;
   return slot_rows(vy, ncols_x, stride_col_y, b, ap) &&
-         dispatch(type, out_type, vx_gate, vx_up, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);
+         dispatch_kq(type, out_type, vx_gate, vx_up, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);
+}
+
+bool qmm_skinny_b32(int type, int out_type, const void *vx, const void *vx2, const void *vy, void *dst, int ncols_x,
+                    int nrows_x, int stride_col_y, int stride_col_dst, int b, int activation, hipStream_t s) {
+  // whole superblocks of eight blocks, and rows that start on dwords
+  if (b < 1 || ncols_x % 256 != 0 || stride_col_y % 2 != 0 || ((uintptr_t)vx | (uintptr_t)vx2 | (uintptr_t)vy) % 4 != 0 ||
+      (int64_t)b * stride_col_y * 34 > 0x7ffffff0)
+    return false;
+  const uint32_t rb = (uint32_t)stride_col_y * 34;
+  const act_rows ap{(const uint8_t *)vy, (int64_t)b * rb, 0, rb, 272, 0, 0, 0};
+  return dispatch_b32(type, out_type, vx, vx2, ap, dst, ncols_x, nrows_x, stride_col_dst, b, activation, s);
 }
 
 // rows of K / 256 blocks of 260 bytes {f32 d; int8 qs[256]}
@@ -424,7 +513,7 @@ bool qmm_skinny_tc(int type, int out_type, const void *vx, const void *vy, void 
   const int64_t rb = (int64_t)(ncols_x / 256) * 260;
   if (b < 1 || b > 32 || ncols_x % 256 != 0 || b * rb > 0x7ffffff0) return false;
   const act_rows ap{(const uint8_t *)vy, b * rb, 4, (uint32_t)rb, 260, 0, (uint32_t)rb, 260};
-  return dispatch(type, out_type, vx, nullptr, ap, dst, ncols_x, nrows_x, stride_col_dst, b, 0, s);
+  return dispatch_kq(type, out_type, vx, nullptr, ap, dst, ncols_x, nrows_x, stride_col_dst, b, 0, s);
 }
 
 // Prefill tiles of one channel: qs[nsb][rows][256] int8, then d[nsb][rows] f32

@@ -65,6 +65,46 @@ def test_glu_rows_over_tile_counts(gtype, per_cu, extra, k, cus):
         assert_parity(got, want, what=f"glu {gtype} n={n} k={k} b={b}")
 
 
+ROWS16 = [O.Q8_0, O.Q4_0, O.Q5_0, O.Q5K]  # the types that take up to 16 rows
+
+
+@pytest.mark.parametrize("gtype", ROWS16)
+@pytest.mark.parametrize("per_cu,extra,k", [(0, 5, 2304), (0, 21, 256), (1, 3, 768), (2, 9, 256), (4, 17, 256)])
+def test_sixteen_row_types_over_tile_counts(gtype, per_cu, extra, k, cus):
+    """Both sides of the row counts from which the kernel takes over, weights that start on a dword only, and all output
+    types (f16 / bf16 within their rounding of the f32 result)."""
+    rng = np.random.default_rng(7400 + per_cu + k)
+    n = 16 * per_cu * cus + extra
+    wq = O.quantize(gtype, weights(rng, n, k))
+    wd = dev(wq, 0 if gtype == O.Q5K else 4)
+    for b in (3, 5, 9, 16):
+        x = acts(rng, b, k)
+        x[b - 1] = 0.0
+        got = qmm.qmatmul_decode(gtype, wd, torch.from_numpy(x).cuda(), n)
+        term = terms(gtype, x, wq, n) if n < 1000 else None
+        assert_parity(got.cpu().numpy(), O.matmul(gtype, x, wq, n), term, what=f"{gtype} n={n} k={k} b={b}")
+        vy, kp = qmm.quantize_decode(gtype, torch.from_numpy(x).cuda())
+        for dt in (torch.float16, torch.bfloat16):
+            assert torch.equal(qmm.mmvq(gtype, wd, vy, k, n, b, kp, out_dtype=dt), got.to(dt))
+
+
+@pytest.mark.parametrize("gtype", ROWS16[:3])
+@pytest.mark.parametrize("n,k", [(19, 1280), (4101, 256)])
+def test_fused_forms_of_32_value_types(gtype, n, k):
+    rng = np.random.default_rng(7500 + n)
+    g, u, v = (O.quantize(gtype, weights(rng, n - 3 * i, k)) for i in range(3))
+    for b in (2, 3, 5, 8, 16):
+        x = acts(rng, b, k)
+        vy, kp = qmm.quantize_decode(gtype, torch.from_numpy(x).cuda())
+        n1 = n - 3  # the up rows past n1 are the next matrix's: not read
+        got = qmm.mmvq_fused_glu(gtype, dev(g), dev(u), vy, k, n1, b, kp).cpu().numpy()
+        want = silu(O.matmul(gtype, x, g, n)[:, :n1]) * O.matmul(gtype, x, u, n1)
+        assert_parity(got, want, what=f"glu {gtype} n={n1} b={b}")
+        qkv = qmm.mmvq_fused_qkv(gtype, dev(g), dev(u), dev(v), vy, k, n, n - 3, n - 6, b, kp)
+        for o, w, m in zip(qkv, (g, u, v), (n, n - 3, n - 6)):
+            assert_parity(o.cpu().numpy(), O.matmul(gtype, x, w, m), what=f"qkv {gtype} n={m} b={b}")
+
+
 @pytest.mark.parametrize("gtype", [O.Q4K, O.Q6K])
 @pytest.mark.parametrize("counts", [(0, 1, 16, 17, 33, 5), (3, 0, 2), (70, 1, 0, 16)])
 def test_grouped_rows_per_expert(gtype, counts):
