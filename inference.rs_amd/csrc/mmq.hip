@@ -1,4 +1,4 @@
-// Prefill matmul for GGUF Q4_K / Q6_K / Q8_0 weights against activations quantized to Q8_K / Q8_0 blocks,
+// Prefill matmul for GGUF weights (K-quants; 32-value blocks Q8_0 / Q4_0 / Q5_0) against activations quantized to Q8_K / Q8_0 blocks,
 // on CDNA4 int8 MFMA (v_mfma_i32_32x32x32_i8), plus its expert-grouped MoE form.
 //
 // Replaces the llama.cpp-derived MMQ of crates/inference-quant/kernels/cuda/mmq_gguf (mmq_instance.cuh:8-268,
@@ -1249,9 +1249,9 @@ __global__ __launch_bounds__(256) void k_mmq_q8_0_moe(const uint8_t *__restrict_
                              nsb, dst, ldd, ids_dst);
 }
 
-// The pipelined 32-value-block kernels: 32 or 64 activation rows per workgroup, two waves per SIMD.
+// The pipelined 32-value-block kernels: 32, 64 or 96 activation rows per workgroup at two waves per SIMD, 128 at one.
 template <int TMv>
-constexpr int b32_waves() { return 2; }
+constexpr int b32_waves() { return TMv == 4 ? 1 : 2; }
 
 template <class WR, class Out, int TMv, bool F32D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(b32_waves<TMv>()))) void k_mmq_b32(
@@ -1334,7 +1334,7 @@ struct KqForm {
 // 133 and 86 (four planes).
 template <class WT>
 constexpr KqForm kq_form(int i) {
-  constexpr bool q4 = WT::kMin && WT::kPlanes == 2, q5 = WT::kPlanes == 3, q6 = WT::kBytes == 210;
+  constexpr bool q4 = WT::kMin && WT::kPlanes == 2, q6 = WT::kBytes == 210;
   return i == 0   ? KqForm{1, 128, 2, false, 2.2}  // up to 32 rows; Q5_K at any
          : i == 1 ? KqForm{2, 128, q4 ? 2 : 1, false, q4 ? 2.4 : q6 ? 3.9 : 1.7}
          : i == 2 ? KqForm{4, 128, 1, false, q6 ? 3.5 : 3.15}
@@ -1348,35 +1348,48 @@ inline double kq_us(const KqForm &f, int64_t tiles, int64_t splits, int64_t nsb,
          (splits > 1 ? 3 + 1.5e-6 * (double)(splits * rows * cols) : 0);
 }
 
+// A form with its tiles and splits of K.  consider() takes form c over what is held when the model's time for it is below
+// `one` times that of the launch the choice started from, with K split below `more` times (the planes' cost is the less
+// certain part) and at least `least` superblocks a split.
+struct KqPlan {
+  KqForm f;
+  int64_t tiles, splits, nsb, rows, cols, planes;  // planes: what the fixup buffer holds
+  double start, best;
+  KqPlan(const KqForm &form, int64_t nsb_, int64_t rows_, int64_t cols_, const void *fixup, int nsm)
+      : f(form), nsb(nsb_), rows(rows_), cols(cols_) {
+    const int cus = qmm_device_cus();
+    tiles = qmm_ceil_div(rows, 32 * f.tm) * qmm_ceil_div(cols, f.cols);
+    splits = k_splits(tiles, nsb, rows, cols, fixup, nsm < cus ? nsm : cus);
+    planes = fixup && (uintptr_t)fixup % 16 == 0 ? (int64_t)(nsm > 0 ? nsm : cus) * 65536 / (4 * rows * cols) : 1;
+    start = best = kq_us(f, tiles, splits, nsb, rows, cols);
+  }
+  void consider(const KqForm &c, double one, double more, int least) {
+    const int64_t t = qmm_ceil_div(rows, 32 * c.tm) * qmm_ceil_div(cols, c.cols);
+    for (int64_t sp = 1; sp == 1 || (sp <= planes && nsb / sp >= least); sp *= 2) {
+      const double us = kq_us(c, t, sp, nsb, rows, cols);
+      if (us < best && us < (sp == 1 ? one : more) * start && (sp - 1) * qmm_ceil_div(nsb, sp) < nsb) {
+        f = c;
+        tiles = t;
+        splits = sp;
+        best = us;
+      }
+    }
+  }
+};
+
 template <class WT, class Out, bool S16 = false>
 void launch_kq(const uint8_t *w, int64_t nrows_x, int64_t w_row_bytes, const ActTile &a, int64_t ncols_y, int64_t nsb,
                typename Out::T *d, int64_t ldd, void *fixup, int nsm, hipStream_t s) {
   // without the wide kernel, the smallest of 32, 64, 128 activation rows that covers the batch, split over as many planes
   // as the reference's fixup buffer holds
-  KqForm f = kq_form<WT>(ncols_y <= 32 || kq_tm_max<WT>() < 2 ? 0 : ncols_y <= 64 || kq_tm_max<WT>() < 4 ? 1 : 2);
-  int64_t tiles = qmm_ceil_div(ncols_y, 32 * f.tm) * qmm_ceil_div(nrows_x, f.cols);
-  int64_t splits = k_splits(tiles, nsb, ncols_y, nrows_x, fixup, nsm < qmm_device_cus() ? nsm : qmm_device_cus());
+  KqPlan plan(kq_form<WT>(ncols_y <= 32 || kq_tm_max<WT>() < 2 ? 0 : ncols_y <= 64 || kq_tm_max<WT>() < 4 ? 1 : 2), nsb,
+              ncols_y, nrows_x, fixup, nsm);
   if (ncols_y > 32) {
-    double best = kq_us(f, tiles, splits, nsb, ncols_y, nrows_x);
-    const int64_t planes = fixup && (uintptr_t)fixup % 16 == 0
-                               ? (int64_t)(nsm > 0 ? nsm : qmm_device_cus()) * 65536 / (4 * ncols_y * nrows_x)
-                               : 1;
-    // (a split wide form only where the model is clear: its planes' cost is the less certain part)
-    const double one = 0.97 * best, more = 0.9 * best;
-    for (int i = 3; i <= 4; i++) {
-      const KqForm c = kq_form<WT>(i);
-      const int64_t t = qmm_ceil_div(ncols_y, 32 * c.tm) * qmm_ceil_div(nrows_x, c.cols);
-      for (int64_t sp = 1; sp == 1 || (sp <= planes && nsb / sp >= 4); sp *= 2) {
-        const double us = kq_us(c, t, sp, nsb, ncols_y, nrows_x);
-        if (us < best && us < (sp == 1 ? one : more) && (sp - 1) * qmm_ceil_div(nsb, sp) < nsb) {
-          f = c;
-          tiles = t;
-          splits = sp;
-          best = us;
-        }
-      }
-    }
+    plan.consider(kq_form<WT>(3), 0.97, 0.9, 4);
+    plan.consider(kq_form<WT>(4), 0.97, 0.9, 4);
   }
+  const KqForm &f = plan.f;
+  const int64_t tiles = plan.tiles, splits = plan.splits;
   float *part = splits > 1 ? (float *)fixup : nullptr;
   const dim3 grid((unsigned)(tiles * splits));
   typedef typename Wide<WT>::T WW;
@@ -1402,17 +1415,38 @@ bool b32_runs(const void *x, int64_t ncols_x, int64_t w_row_bytes) {
   return ncols_x % 256 == 0 && w_row_bytes % 4 == 0 && (uintptr_t)x % 4 == 0;
 }
 
+// The same model's forms of the 32-value types: a weight block is decoded once for 32 tm activation rows; the LDS slots of
+// up to 96 rows leave room for two workgroups per CU.  Measured on MI355X, us, 64 / 96 / 128 rows: 8192x4096 at 333 rows
+// Q4_0 63.6 / 53.6 / 63.6, Q8_0 70 / 64.5 / 78.8, Q5_0 68 / 54.9 / 67.0; 11008x4096 at 1024 rows Q4_0 157 / 147 / 183, Q8_0
+// 184 / 169 / 228; 14336x4096 at 512 rows Q4_0 112-121 / 112 / 123; 4096x14336 at 512 rows, the last two in two splits of
+// K, Q4_0 114 / 129 / 109, Q8_0 157 / 144 / 135, Q5_0 130 / 140 / 117 (64 rows in two splits Q8_0 114, Q4_0 103).
+template <class WR>
+constexpr KqForm b32_form(int tm) {
+  constexpr bool q4 = WR::kBytes == 18, q8 = WR::kBytes == 34;
+  return tm == 1   ? KqForm{1, BN, 2, false, 2.2}
+         : tm == 2 ? KqForm{2, BN, 2, false, q4 ? 3.6 : q8 ? 4.4 : 3.95}
+         : tm == 3 ? KqForm{3, BN, 2, false, q4 ? 4.5 : q8 ? 5.5 : 4.8}
+                   : KqForm{4, BN, 1, false, q4 ? 3.6 : q8 ? 4.4 : 3.8};
+}
+
 template <class WR, class Out, bool F32D>
 void launch_b32(const uint8_t *w, int64_t nrows_x, int64_t w_row_bytes, const ActTile &a, int64_t ncols_y,
                 int64_t nsb, typename Out::T *d, int64_t ldd, void *fixup, int nsm, hipStream_t s) {
-  const int64_t ntiles = (nrows_x + BN - 1) / BN;
-  const int tm = ncols_y <= 32 ? 1 : 2;
-  const int64_t tiles = ((ncols_y + 32 * tm - 1) / (32 * tm)) * ntiles;
-  const int64_t splits = k_splits(tiles, nsb, ncols_y, nrows_x, fixup, nsm);
+  // 32 activation rows up to 32 rows, 64 up to 64; above, 64, 96 or 128 by the model.  (At 0.97 a second look at random
+  // shapes found 128 rows slower at 14215x1536, 475 rows, Q5_0 57.4 and 51.9 us, 96 at 12495x8448, 744 rows, Q4_0 270 and
+  // 256, and short splits at 1641x4864, 635 rows, Q8_0 58.7 and 54.4: hence the limits.)
+  KqPlan plan(b32_form<WR>(ncols_y <= 32 ? 1 : 2), nsb, ncols_y, nrows_x, fixup, nsm);
+  if (ncols_y > 64)
+    for (int tm = 2; tm <= 4; tm++) plan.consider(b32_form<WR>(tm), 0.93, 0.92, 12);
+  const int64_t splits = plan.splits;
   float *part = splits > 1 ? (float *)fixup : nullptr;
-  const dim3 grid((unsigned)(tiles * splits));
-  if (tm == 1)
+  const dim3 grid((unsigned)(plan.tiles * splits));
+  if (plan.f.tm == 1)
     k_mmq_b32<WR, Out, 1, F32D><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
+  else if (plan.f.tm == 3)
+    k_mmq_b32<WR, Out, 3, F32D><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
+  else if (plan.f.tm == 4)
+    k_mmq_b32<WR, Out, 4, F32D><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
   else
     k_mmq_b32<WR, Out, 2, F32D><<<grid, 256, 0, s>>>(w, nrows_x, w_row_bytes, a, ncols_y, nsb, splits, d, ldd, part);
   if (part) split_sum<Out>(part, splits, ncols_y, nrows_x, d, ldd, nullptr, s);

@@ -203,3 +203,26 @@ def test_wide_prefill_split_k(gtype, n, k, m):
         H.qmm_qtensor_free(h)
     assert torch.equal(outs[0], outs[1])
     assert_parity(outs[0].cpu().numpy(), O.matmul(gtype, x, wq, n), what=f"split wide {gtype} n={n} k={k} m={m}")
+
+
+@pytest.mark.parametrize("gtype", ROWS16[:3])
+@pytest.mark.parametrize("n,k,m", [(16583, 1280, 90), (16583, 1280, 121), (16640, 256, 96), (4019, 14336, 470)])
+def test_prefill_tiles_of_32_value_types(gtype, n, k, m):
+    """96- and 128-row activation tiles with ragged rows and weight rows (more weight tiles than half the compute units),
+    and the shape where K is split; both activation layouts.  A prime count of distinct weight rows repeats, so that a
+    misplaced tile shows.  f16 output is the f32 one rounded."""
+    rng = np.random.default_rng(7600 + n + m)
+    u = 67
+    wq = O.quantize(gtype, weights(rng, u, k))
+    rows = np.arange(n) % u
+    wd = dev(np.ascontiguousarray(wq).reshape(-1).view(np.uint8).reshape(u, -1)[rows])
+    x = acts(rng, m, k)
+    xd = torch.from_numpy(x).cuda()
+    y, _ = qmm.quantize_prefill(gtype, xd)
+    got = qmm.mmq(gtype, wd, y, k, n, m)
+    assert_parity(got.cpu().numpy(), O.matmul(gtype, x, wq, u)[:, rows], what=f"{gtype} {n}x{k} m={m}")
+    assert torch.equal(qmm.mmq(gtype, wd, y, k, n, m, out_dtype=torch.float16), got.half())
+    y, _ = qmm.quantize_prefill(gtype, xd, q8_1=True)
+    got = qmm.mmq(gtype, wd, y, k, n, m, q8_1=True)
+    one = qmm.mmq(gtype, wd, y, k, n, m, q8_1=True, tmp_fixup=False)  # K in one piece
+    assert (got - one).abs().max() <= 1e-5 * one.abs().max()
